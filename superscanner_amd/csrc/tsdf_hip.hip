@@ -1363,13 +1363,18 @@ void k_raycast(GridView g, Pose pose, RayParams rp, float* points, float* colors
     }
     unsigned int hit = 0, bad = 0, samples = 0, probes = 0;
     // the depth bound of this wavefront's 8 x 8 pixels (one tile of the map)
-    float zt = -1.0f;
-    if (rq.use_tb && tile < n_tiles)
-        zt = tb_depth(tb.z[(size_t)(i / kTbTile) * tb.tiles_x + (j / kTbTile)], tb.epoch);
+    float zt = -1.0f, zf = -1.0f;
+    if (rq.use_tb && tile < n_tiles) {
+        // (the last tile's wavefronts may lie past the image's 8 x 8 tiles)
+        const int ty = min(i / kTbTile, tb.tiles_y - 1), tx = min(j / kTbTile, tb.tiles_x - 1);
+        zt = tb_depth(tb.z[(size_t)ty * tb.tiles_x + tx], tb.epoch);
+        const int fy = min(i / kTbFarTile, tb.far_y - 1), fx = min(j / kTbFarTile, tb.far_x - 1);
+        zf = tb_far(tb.zf[(size_t)fy * tb.far_x + fx], tb.epoch);
+    }
     RayState st;
     bool defer = false;
     if (tile < n_tiles && i < rp.H && j < rp.W) {
-        const RayResult r = march<T, kColor, kStats>(g, pose, rq, i, j, fp, zt, kStats ? 0 : rq.budget, &st);
+        const RayResult r = march<T, kColor, kStats>(g, pose, rq, i, j, fp, zt, kStats ? 0 : rq.budget, &st, zf);
         defer = r.code == kRayDeferred;
         if (!defer) {
             write_ray(r, (size_t)i * rp.W + j, pose, points, colors, depth, ub);
@@ -1414,11 +1419,15 @@ void k_raycast(GridView g, Pose pose, RayParams rp, float* points, float* colors
 // k_ray_bounds: the tile depth bounds of one raycast (TileBounds in
 // tsdf_march.hpp).  A workgroup takes a contiguous run of brick ids (bricks
 // allocated together are spatial neighbours, so a run covers few tiles),
-// lowers the bounds of the tiles each grown brick may cover in a copy of the
-// tile map in LDS, then merges its copy into the global map with one atomic
-// per tile it touched.  Larger images than kTbLdsTiles tiles lower the global
-// map directly.
-constexpr int kTbLdsTiles = 16384;  // 64 KiB of LDS: 1280 x 720 has 14 400 tiles
+// lowers the near bounds and raises the far bounds of the tiles each grown
+// brick may cover in a copy of the tile maps in LDS, then merges its copy into
+// the global maps with one atomic per tile it touched.  Larger images than
+// kTbLdsTiles tiles go to the global maps directly.
+// Bound by a fixed chain (clear the copy, load, project, merge), 15 us at
+// 848 x 480 and 47 us at 1280 x 720 over 650 k bricks; the far bound, at a
+// quarter of the tiles, costs 1 and 5 us of it and ends every ray that
+// leaves the map (160 x 120 over an open plane: raycast 447 -> 159 us).
+constexpr int kTbLdsTiles = 16384;  // 80 KiB of LDS: 1280 x 720 has 14 400 tiles, and two copies fit a CU
 #ifndef TSDF_TB_PER
 #define TSDF_TB_PER 128  // least bricks per workgroup run
 #endif
@@ -1432,50 +1441,88 @@ __device__ __forceinline__ uint32_t f32_bits(float f)
     return __float_as_uint(f);
 }
 
+__host__ __device__ __forceinline__ int pad4(int n) { return (n + 3) & ~3; }
+
+// Lowers / raises the bounds of the tiles that bricks [0, alloc_top) may
+// cover in an H x W image with pose P; block `wg` of `n_wg`.
 template <bool kLds>
-__global__ __launch_bounds__(kThreads) void k_ray_bounds(GridView g, Pose P, TileBounds tb)
+__device__ void bounds_block(const GridView& g, const Pose& P, const Camera& cam, int H, int W, const TileBounds& tb,
+                             unsigned int wg, unsigned int n_wg)
 {
-    extern __shared__ uint32_t lz[];  // [tiles] positive depths compare as their bits
+    extern __shared__ __align__(16) uint32_t lz[];  // [tiles] least, [far tiles] greatest: positive depths compare as bits
     // the allocated count is known only here: runs of at least TSDF_TB_PER
     // bricks, the workgroups past the last run leave at once
     const unsigned int n = min(g.ctrl->alloc_top, g.n_bricks);
-    const unsigned int per = max((n + gridDim.x - 1) / gridDim.x, (unsigned int)TSDF_TB_PER);
-    const unsigned int b0 = blockIdx.x * per, b1 = min(n, b0 + per);
+    const unsigned int per = max((n + n_wg - 1) / n_wg, (unsigned int)TSDF_TB_PER);
+    const unsigned int b0 = wg * per, b1 = min(n, b0 + per);
     if (b0 >= n)
         return;
-    const int nt = tb.tiles_x * tb.tiles_y;
+    const int nt = pad4(tb.tiles_x * tb.tiles_y), nf = pad4(tb.far_x * tb.far_y);
+    uint32_t* lf = lz + nt;
     if (kLds) {
-        for (int t = threadIdx.x; t < nt; t += kThreads)
-            lz[t] = kTbNone;
+        // four words at a time (lz is padded to a multiple of four)
+        uint4* q = (uint4*)lz;
+        for (int t = threadIdx.x; t < nt / 4; t += kThreads)
+            q[t] = make_uint4(kTbNone, kTbNone, kTbNone, kTbNone);
+        q = (uint4*)lf;
+        for (int t = threadIdx.x; t < nf / 4; t += kThreads)
+            q[t] = make_uint4(0u, 0u, 0u, 0u);
         __syncthreads();
     }
     for (unsigned int id = b0 + threadIdx.x; id < b1; id += kThreads) {
         const int4 c = g.coords[id];
-        float zmin;
+        float zmin, zmax;
         int r0, r1, c0, c1;
-        if (!brick_bounds(c.x, c.y, c.z, g.vbl, P, g.cam, g.H, g.W, tb.grow, tb.z_lo, zmin, r0, r1, c0, c1))
+        if (!brick_span(c.x, c.y, c.z, g.vbl, P, cam, H, W, tb.grow, tb.z_lo, zmin, zmax, r0, r1, c0, c1))
             continue;
-        const uint32_t zb = f32_bits(zmin);
+        const uint32_t zb = f32_bits(zmin), fb = f32_bits(zmax);
         for (int ty = r0 / kTbTile; ty <= r1 / kTbTile; ++ty)
             for (int tx = c0 / kTbTile; tx <= c1 / kTbTile; ++tx) {
                 if (kLds) {
                     uint32_t* q = &lz[ty * tb.tiles_x + tx];
                     if (*q > zb)  // most bricks lie behind a nearer one of the tile
                         atomicMin(q, zb);
-                }
-                else
+                } else {
                     atomicMin(tb.z + (size_t)ty * tb.tiles_x + tx, tb_pack(tb.epoch, zmin));
+                }
+            }
+        for (int ty = r0 / kTbFarTile; ty <= r1 / kTbFarTile; ++ty)
+            for (int tx = c0 / kTbFarTile; tx <= c1 / kTbFarTile; ++tx) {
+                if (kLds) {
+                    uint32_t* q = &lf[ty * tb.far_x + tx];
+                    if (*q < fb)
+                        atomicMax(q, fb);
+                } else {
+                    atomicMax(tb.zf + (size_t)ty * tb.far_x + tx, tb_pack_far(tb.epoch, zmax));
+                }
             }
     }
     if (kLds) {
         __syncthreads();
-        const unsigned long long hi = (unsigned long long)(~tb.epoch) << 32;
-        for (int t = threadIdx.x; t < nt; t += kThreads) {
-            const uint32_t v = lz[t];
-            if (v != kTbNone)
-                atomicMin(tb.z + t, hi | v);
+        const unsigned long long hi = (unsigned long long)(~tb.epoch) << 32, hf = (unsigned long long)tb.epoch << 32;
+        for (int t = threadIdx.x; t < nt / 4; t += kThreads) {
+            const uint4 v = ((const uint4*)lz)[t];
+            const uint32_t e[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                if (e[k] != kTbNone)  // never so in the padding
+                    atomicMin(tb.z + 4 * t + k, hi | e[k]);
+        }
+        for (int t = threadIdx.x; t < nf / 4; t += kThreads) {
+            const uint4 v = ((const uint4*)lf)[t];
+            const uint32_t e[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                if (e[k])
+                    atomicMax(tb.zf + 4 * t + k, hf | e[k]);
         }
     }
+}
+
+template <bool kLds>
+__global__ __launch_bounds__(kThreads) void k_ray_bounds(GridView g, Pose P, TileBounds tb)
+{
+    bounds_block<kLds>(g, P, g.cam, g.H, g.W, tb, blockIdx.x, gridDim.x);
 }
 
 // The slowest-first tile order for the next raycast: tiles sorted by the
@@ -1621,7 +1668,8 @@ struct tsdf_grid {
     Ctrl* ctrl_host;  // pinned
     unsigned long long* stat;       // statistics counters, kStatWords
     unsigned long long* stat_host;  // pinned
-    unsigned long long* tb_z;       // [8x8-pixel tiles] depth bounds of the raycasts (TileBounds)
+    unsigned long long* tb_z;       // [8x8-pixel tiles] least and greatest depths of the raycasts (TileBounds)
+    unsigned long long* tb_zf;
     RayState* ray_queue;            // [H * W] rays a raycast deferred to its tail kernel
     uint32_t ray_qepoch;            // raycasts that used the queue (their parity picks the counters)
     uint32_t tb_epoch;
@@ -1906,8 +1954,11 @@ TileBounds tile_bounds(tsdf_grid* g, const Pose& P)
 {
     TileBounds tb;
     tb.z = g->tb_z;
+    tb.zf = g->tb_zf;
     tb.tiles_x = (g->p.width + kTbTile - 1) / kTbTile;
     tb.tiles_y = (g->p.height + kTbTile - 1) / kTbTile;
+    tb.far_x = (g->p.width + kTbFarTile - 1) / kTbFarTile;
+    tb.far_y = (g->p.height + kTbFarTile - 1) / kTbFarTile;
     tb.epoch = g->tb_epoch;
     const double vl = g->p.voxel_length, dt = g->p.truncation, vbl = g->vbl, dmax = g->p.max_ray_length;
     const double n_upd = 4.0 * (dmax + vbl) / (vl < dt ? vl : dt) + 64.0;
@@ -1952,6 +2003,20 @@ void launch_raycast(tsdf_grid* g, const Pose& P, float* points, float* colors, f
     rp.use_tb = g->tune.raycast_skip == 2 && !kStats;
     // the group march replays no superblock distance field
     rp.budget = (kStats || rp.use_sb) ? 0 : g->tune.raycast_budget;
+    // How readily a ray is deferred.  One round of the 16-lane march looks up
+    // 16 positions of a ray with 16 lanes' work, the per-lane march 4 with
+    // one, so deferring pays by itself only in a wavefront with few rays left
+    // (16 lanes), and everywhere while the chip has lanes to spare.  What it
+    // has to do is bounded by the lookups of an empty march, wavefronts x
+    // d_max / vbl.  Raycast with 16 / 16, 16 / 64 and 64 / 64 lanes (run / top):
+    //   575 k  (320 x 180, 16 mm bricks)   537   541  358 us
+    //   1.2 M  (640 x 480, 40 mm)          244   226  226
+    //   2.0 M  (848 x 480, 32 mm)          206   186  185
+    //   2.25 M (640 x 360, 16 mm)          854   893 1005
+    //   9.0 M  (1280 x 720, 16 mm)        1654  1865 3389
+    const double lookups = (double)((rp.W + 7) / 8) * ((rp.H + 7) / 8) * (rp.dmax / rp.vbl);
+    rp.defer_run = lookups < 0.8e6 ? 64 : 16;
+    rp.defer_top = lookups < 2.1e6 ? 64 : 16;
     rp.lc = nullptr;  // the kernel points it at its LDS cache (TSDF_RAY_CACHE)
     const int qpar = (int)(g->ray_qepoch & 1u);
     if (rp.budget > 0)
@@ -1972,8 +2037,8 @@ void launch_raycast(tsdf_grid* g, const Pose& P, float* points, float* colors, f
         tb.epoch = ++g->tb_epoch;
         const int nt = tb.tiles_x * tb.tiles_y;
         if (nt <= kTbLdsTiles && !TSDF_TB_GLOBAL)
-            hipLaunchKernelGGL((k_ray_bounds<true>), dim3(g->n_cu * 4), dim3(kThreads), (size_t)nt * sizeof(uint32_t),
-                               s, view(g), P, tb);
+            hipLaunchKernelGGL((k_ray_bounds<true>), dim3(g->n_cu * 4), dim3(kThreads),
+                               (size_t)(pad4(nt) + pad4(tb.far_x * tb.far_y)) * sizeof(uint32_t), s, view(g), P, tb);
         else
             hipLaunchKernelGGL((k_ray_bounds<false>), dim3(g->n_cu * 4), dim3(kThreads), 0, s, view(g), P, tb);
     }
@@ -2169,10 +2234,13 @@ tsdf_status tsdf_create(const tsdf_params* p, tsdf_grid** out)
         alloc((void**)&g->ray_order, tiles * sizeof(uint32_t));
         const size_t t8 = (size_t)((p->width + kTbTile - 1) / kTbTile) * ((p->height + kTbTile - 1) / kTbTile);
         alloc((void**)&g->tb_z, t8 * sizeof(unsigned long long));
+        alloc((void**)&g->tb_zf, t8 * sizeof(unsigned long long));
         alloc((void**)&g->ray_queue, (size_t)p->width * p->height * sizeof(RayState));
         if (st == TSDF_OK) {
             // no entry carries an epoch yet (epochs start at 1, ~1 != ~0)
             hipError_t e = hipMemset(g->tb_z, 0xFF, t8 * sizeof(unsigned long long));
+            if (e == hipSuccess)
+                e = hipMemset(g->tb_zf, 0, t8 * sizeof(unsigned long long));
             if (e != hipSuccess)
                 st = fail(TSDF_HIP_ERROR, std::string("hipMemset: ") + hipGetErrorString(e));
         }
@@ -2237,6 +2305,7 @@ void tsdf_destroy(tsdf_grid* g)
     (void)hipFree(g->ray_cost);
     (void)hipFree(g->ray_order);
     (void)hipFree(g->tb_z);
+    (void)hipFree(g->tb_zf);
     (void)hipFree(g->ray_queue);
     (void)hipFree(g->op_mask);
     (void)hipFree(g->ptmap_batch);

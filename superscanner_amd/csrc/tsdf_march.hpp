@@ -135,6 +135,8 @@ __host__ __device__ __forceinline__ int find_brick(const GridView& g, int x, int
 // Probe result from the first slot word alone: the id, -1 (absent), or
 // kProbeMore when the slot holds another key and probing must continue.
 constexpr int kProbeMore = -2;
+// probe_run stopped at its round budget, the next lookup not yet made.
+constexpr int kProbeDeferred = -3;
 __host__ __device__ __forceinline__ int first_slot(const GridView& g, uint32_t key, unsigned long long s)
 {
     const uint32_t id = (uint32_t)s;
@@ -283,6 +285,7 @@ struct RayParams {
     int df_lo[3], df_dim[3];
     int use_tb;       // tile depth bounds replay allowed (alias certificate holds)
     int budget;       // rounds of the per-lane march before a ray is deferred (0: never)
+    int defer_run, defer_top;  // most lanes still in a probing run / in the march for a deferral there
     unsigned long long* lc;  // the workgroup's LDS cache of lookup results, or null
 };
 
@@ -356,15 +359,23 @@ __host__ __device__ __forceinline__ void cache_result(const RayParams& rp, uint3
 // map needs no clearing: an entry is (~epoch << 32) | bits(depth) under
 // atomicMin, so this raycast's entries are below every older one and a tile
 // without one reads as empty (every lookup of its rays misses).
+//
+// The far bound is the mirror image: each 16 x 16-pixel tile keeps the
+// greatest camera depth of the grown boxes that touch it ((epoch << 32) | bits under
+// atomicMax).  Beyond it no brick holds a position of the tile's rays, so
+// every later lookup misses too.
 // ---------------------------------------------------------------------------
 #ifndef TSDF_TB_TILE
 #define TSDF_TB_TILE 8
 #endif
 constexpr int kTbTile = TSDF_TB_TILE;  // tile side in pixels: the 8 x 8 pixels of a raycast wavefront
+constexpr int kTbFarTile = 2 * TSDF_TB_TILE;  // of the far bound, which need not be as tight
 
 struct TileBounds {
-    unsigned long long* z;  // [tiles_y * tiles_x]
+    unsigned long long* z;   // [tiles_y * tiles_x] least depth
+    unsigned long long* zf;  // [far_y * far_x] greatest depth
     int tiles_x, tiles_y;
+    int far_x, far_y;
     uint32_t epoch;
     float grow;  // metres a brick box grows by
     float z_lo;  // least depth of a probe-run position
@@ -378,6 +389,27 @@ __host__ __device__ __forceinline__ unsigned long long tb_pack(uint32_t epoch, f
     } b;
     b.f = z;
     return ((unsigned long long)(~epoch) << 32) | b.u;
+}
+
+__host__ __device__ __forceinline__ unsigned long long tb_pack_far(uint32_t epoch, float z)
+{
+    union {
+        float f;
+        uint32_t u;
+    } b;
+    b.f = z;
+    return ((unsigned long long)epoch << 32) | b.u;
+}
+
+// The far bound of this raycast (epoch), 0 for a tile no brick touched.
+__host__ __device__ __forceinline__ float tb_far(unsigned long long e, uint32_t epoch)
+{
+    union {
+        float f;
+        uint32_t u;
+    } b;
+    b.u = (uint32_t)e;
+    return (uint32_t)(e >> 32) == epoch ? b.f : 0.0f;
 }
 
 // The tile bound of this raycast (epoch), +inf for a tile no brick touched.
@@ -404,11 +436,11 @@ __host__ __device__ __forceinline__ float approx_rcp(float z)
 
 // Bounds of brick (bx, by, bz): false when no probe-run position can lie in
 // it (all of it nearer than z_lo, or outside the image), else its least
-// depth beyond z_lo and the inclusive pixel range [r0, r1] x [c0, c1] its
-// grown box may cover.
-__host__ __device__ __forceinline__ bool brick_bounds(int bx, int by, int bz, float vbl, const Pose& P,
-                                                      const Camera& cam, int H, int W, float grow, float z_lo,
-                                                      float& zmin, int& r0, int& r1, int& c0, int& c1)
+// depth beyond z_lo, its greatest depth and the inclusive pixel range
+// [r0, r1] x [c0, c1] its grown box may cover.
+__host__ __device__ __forceinline__ bool brick_span(int bx, int by, int bz, float vbl, const Pose& P,
+                                                    const Camera& cam, int H, int W, float grow, float z_lo,
+                                                    float& zmin, float& zmax, int& r0, int& r1, int& c0, int& c1)
 {
     const float lo[3] = {vbl * (float)bx - grow, vbl * (float)by - grow, vbl * (float)bz - grow};
     const float hi[3] = {vbl * (float)bx + vbl + grow, vbl * (float)by + vbl + grow, vbl * (float)bz + vbl + grow};
@@ -477,7 +509,17 @@ __host__ __device__ __forceinline__ bool brick_bounds(int bx, int by, int bz, fl
     if (r0 > r1 || c0 > c1)
         return false;
     zmin = z0;
+    zmax = z1;
     return true;
+}
+
+// brick_span without the greatest depth.
+__host__ __device__ __forceinline__ bool brick_bounds(int bx, int by, int bz, float vbl, const Pose& P,
+                                                      const Camera& cam, int H, int W, float grow, float z_lo,
+                                                      float& zmin, int& r0, int& r1, int& c0, int& c1)
+{
+    float zmax;
+    return brick_span(bx, by, bz, vbl, P, cam, H, W, grow, z_lo, zmin, zmax, r0, r1, c0, c1);
 }
 
 // The ray parameter below which every lookup of ray (i, j) misses: the
@@ -489,6 +531,14 @@ __host__ __device__ __forceinline__ float tb_l_safe(float zt, float nz, float dm
         return dmax;
     const float l = (zt * (1.0f - 1e-5f) - 1e-5f) / nz;
     return l < dmax ? l : dmax;
+}
+
+// The ray parameter from which every lookup of the ray misses: the tile's far
+// bound, with a margin that need not be tight (what it costs is one more
+// round of lookups).
+__host__ __device__ __forceinline__ float tb_l_far(float zf, float nz)
+{
+    return (zf * (1.0f + 1e-4f) + 1e-4f) / nz;
 }
 
 // The reference's index rule on a quotient q = RN32(a / d) (exact through
@@ -526,20 +576,28 @@ struct RayResult {
     unsigned int samples, probes;
 };
 
-// A march stopped at the top of its outer loop (code kRayDeferred) and
-// resumed later by march_group: its position, length, the last sample's
-// weight sign, the lookup loaded ahead for the next position and the counts
-// so far.  Everything else of the march is recomputed from the pixel.
+// A march stopped at the top of its outer loop or between two rounds of a
+// probing run (code kRayDeferred) and resumed later by march_group: its
+// position, length, the last sample's weight sign, the lookup loaded ahead
+// for the next position and the counts so far.  Everything else of the march
+// is recomputed from the pixel.
 constexpr int kRayDeferred = 2;
+enum RayFlags : uint32_t {
+    kRayLp = 1u,       // the last sample's weight was positive
+    kRayPre = 2u,      // pre_key, pre_bk and pre_slot hold the next lookup
+    kRaySkip = 4u,     // inside the empty-block skip (steps of vbl were taken)
+    kRayAdvance = 8u,  // inside the re-advance by d_trunc
+};
 struct RayState {
     float rx, ry, rz, l;
     uint32_t pix;          // i * W + j
-    uint32_t flags;        // bit 0 Lp, bit 1 pre_valid
+    uint32_t flags;        // RayFlags
     uint32_t pre_key, pre_bk;
     unsigned long long pre_slot;
     uint32_t samples, probes;
     float zt;              // the tile depth bound of the ray (< 0: none)
-    uint32_t pad[3];
+    float zf;              // its tile's far bound (< 0: none)
+    uint32_t pad[2];
 };
 static_assert(sizeof(RayState) == 64, "one 64-byte record per deferred ray");
 
@@ -653,6 +711,16 @@ inline void sbdf_build_host(const uint32_t* sb_bits, const int lo[3], const int 
             }
 }
 
+// Lanes of the wavefront that run this point together (1 on the host).
+__host__ __device__ __forceinline__ int active_lanes()
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __popcll(__ballot(1));
+#else
+    return 1;
+#endif
+}
+
 template <bool kStats>
 __host__ __device__ __forceinline__ int probe_count(const GridView& g, const Footprint& fp, int x, int y, int z,
                                                     unsigned int& probes)
@@ -694,18 +762,23 @@ __host__ __device__ __forceinline__ f3 sel3(bool c, f3 a, f3 b) { return {c ? a.
 //    at most vbl per axis) move the reference's block index by at most k + 3
 //    per axis, so steps 1 .. d - 4 miss.
 // Returns the brick id (>= 0) or -1; steps counts the steps taken, probes
-// every lookup of the reference (replayed ones included).
+// every lookup of the reference (replayed ones included).  l_end <= d_max: the
+// run stops there (no brick holds a position of the ray from l_end on), and
+// the caller counts the misses up to d_max.  With a budget > 0
+// it returns kProbeDeferred once `rounds` reached it, another round would be
+// needed (every lookup so far missed, the next position not yet taken) and at
+// most rp.defer_run lanes of the wavefront are still in the run.
 //
 // pre_valid: the first slot word of the lookup at rv (key pre_key, bucket
 // pre_bk) was already loaded as pre_slot; a hit there costs no further load.
 template <bool kStats>
 __host__ __device__ __forceinline__ int probe_run(const GridView& g, const RayParams& rp, const Footprint& fp, f3& rv,
                                                   float& l, const f3 delta, float dl, int& steps, unsigned int& probes,
-                                                  float l_safe, int& rounds, bool pre_valid = false,
+                                                  float l_safe, float l_end, int& rounds, int budget,
+                                                  bool pre_valid = false,
                                                   uint32_t pre_key = 0, uint32_t pre_bk = 0,
                                                   unsigned long long pre_slot = 0)
 {
-    const float dmax = rp.dmax;
     int id = -1;
     bool first = true;  // the lookup at rv itself has not been made
     if (pre_valid) {
@@ -721,7 +794,7 @@ __host__ __device__ __forceinline__ int probe_run(const GridView& g, const RayPa
     }
     bool have = false;  // nrep holds the replay count for the block of rv
     int nrep = 0;
-    while (first || (id < 0 && l < dmax)) {
+    while (first || (id < 0 && l < l_end)) {
         // tile depth bounds: the lookups at ray parameters below l_safe
         // miss (l_safe <= d_max, so every such miss is followed by a step)
         if (first && l < l_safe) {
@@ -745,16 +818,18 @@ __host__ __device__ __forceinline__ int probe_run(const GridView& g, const RayPa
                 vb3(rv, rp, cx, cy, cz);
                 nrep = free_dist(rp, cx, cy, cz) - 4;
             }
-            for (int k = 0; k < nrep && l < dmax; ++k) {
+            for (int k = 0; k < nrep && l < l_end; ++k) {
                 rv = add3(rv, delta);
                 l += dl;
                 ++steps;
                 ++probes;
             }
             have = false;
-            if (!(l < dmax))
+            if (!(l < l_end))
                 break;
         }
+        if (!first && budget > 0 && rounds >= budget && active_lanes() <= rp.defer_run)
+            return kProbeDeferred;
         // positions: rv itself first (on the first round), then steps
         uint32_t key[kSkipLook], bk[kSkipLook];
         unsigned long long sl[kSkipLook];
@@ -797,7 +872,7 @@ __host__ __device__ __forceinline__ int probe_run(const GridView& g, const RayPa
             pend = pend || more;
             pkey = more ? key[k] : pkey;
             pbk = more ? bk[k] : pbk;
-            go = go && r0 == -1 && l < dmax;
+            go = go && r0 == -1 && l < l_end;
         }
         first = false;
         if (rp.use_sb && go) {  // every lookup taken and missed: rv is the last position
@@ -810,6 +885,16 @@ __host__ __device__ __forceinline__ int probe_run(const GridView& g, const RayPa
         }
     }
     return id;
+}
+
+// The rest of a probing run beyond the last brick: every lookup misses, the
+// ray ends at d_max and only the lookups are counted.
+__host__ __device__ __forceinline__ void miss_to_end(float& l, float dl, float dmax, unsigned int& probes)
+{
+    while (l < dmax) {
+        l += dl;
+        ++probes;
+    }
 }
 
 // The zero crossing, GPUVoxelGrid.cpp:655-689: rv is the first position at
@@ -888,11 +973,12 @@ __host__ __device__ __forceinline__ void ray_setup(const GridView& g, const Pose
 }
 
 // budget > 0: after that many probe rounds and walk windows the march stops
-// at the top of its outer loop, returns kRayDeferred and leaves its state in
-// *st (march_group resumes it).
+// at the top of its outer loop or before the next round of a probing run,
+// returns kRayDeferred and leaves its state in *st (march_group resumes it).
 template <typename T, bool kColor, bool kStats>
 __host__ __device__ RayResult march(const GridView& g, const Pose& pose, const RayParams& rp, int i, int j,
-                                    const Footprint& fp, float zt = -1.0f, int budget = 0, RayState* st = nullptr)
+                                    const Footprint& fp, float zt = -1.0f, int budget = 0, RayState* st = nullptr,
+                                    float zf = -1.0f)
 {
     RayResult out;
     out.p = {0.f, 0.f, 0.f};
@@ -906,6 +992,7 @@ __host__ __device__ RayResult march(const GridView& g, const Pose& pose, const R
     ray_setup(g, pose, i, j, n, rv, dir);
     // the tile bound of this ray's tile (zt < 0: no replay)
     const float l_safe = (rp.use_tb && zt >= 0.0f) ? tb_l_safe(zt, n.z, dmax) : -1.0f;
+    const float l_end = (rp.use_tb && zf >= 0.0f) ? fminf(tb_l_far(zf, n.z), dmax) : dmax;
     float l = 0.1f;
     int rounds = 0;
     const f3 skip = {vbl * dir.x, vbl * dir.y, vbl * dir.z};  // the reference's vbl * dir
@@ -916,29 +1003,27 @@ __host__ __device__ RayResult march(const GridView& g, const Pose& pose, const R
     bool pre_valid = false;
     uint32_t pre_key = 0, pre_bk = 0;
     unsigned long long pre_slot = 0;
+    budget = st ? budget : 0;
+    uint32_t where = 0;  // kRaySkip / kRayAdvance: deferred inside that run
+    bool deferred = false;
     while (l < dmax) {  // outer loop; done / Fn leave by return
-        if (budget > 0 && rounds >= budget && st) {
-            st->rx = rv.x;
-            st->ry = rv.y;
-            st->rz = rv.z;
-            st->l = l;
-            st->pix = (uint32_t)(i * rp.W + j);
-            st->flags = (Lp ? 1u : 0u) | (pre_valid ? 2u : 0u);
-            st->pre_key = pre_key;
-            st->pre_bk = pre_bk;
-            st->pre_slot = pre_slot;
-            st->samples = out.samples;
-            st->probes = out.probes;
-            st->zt = zt;
-            out.code = kRayDeferred;
-            return out;
+        if (budget > 0 && rounds >= budget && active_lanes() <= rp.defer_top) {
+            deferred = true;
+            break;
         }
         // ---- the block lookup at rv and the empty-block skip ------------
         // (GPUVoxelGrid.cpp:589-604): probe rv, then steps of vbl * dir
         int count = 0;
-        int id = probe_run<kStats>(g, rp, fp, rv, l, skip, vbl, count, out.probes, l_safe, rounds, pre_valid,
-                                   pre_key, pre_bk, pre_slot);
+        int id = probe_run<kStats>(g, rp, fp, rv, l, skip, vbl, count, out.probes, l_safe, l_end, rounds, budget,
+                                   pre_valid, pre_key, pre_bk, pre_slot);
         pre_valid = false;
+        if (id == kProbeDeferred) {
+            where = kRaySkip;
+            deferred = true;
+            break;
+        }
+        if (id < 0 && l < dmax)
+            miss_to_end(l, vbl, dmax, out.probes);
         if (!(l < dmax))
             break;
         if (count > 0) {
@@ -951,7 +1036,15 @@ __host__ __device__ RayResult march(const GridView& g, const Pose& pose, const R
             l -= back;
             const f3 dstep = {dt * dir.x, dt * dir.y, dt * dir.z};
             int steps = 0;
-            id = probe_run<kStats>(g, rp, fp, rv, l, dstep, dt, steps, out.probes, l_safe, rounds);
+            id = probe_run<kStats>(g, rp, fp, rv, l, dstep, dt, steps, out.probes, l_safe, l_end, rounds,
+                                   budget);
+            if (id == kProbeDeferred) {
+                where = kRayAdvance;
+                deferred = true;
+                break;
+            }
+            if (id < 0 && l < dmax)
+                miss_to_end(l, dt, dmax, out.probes);
         }
         if (!(l < dmax))
             break;
@@ -1087,6 +1180,22 @@ __host__ __device__ RayResult march(const GridView& g, const Pose& pose, const R
             crossing<T, kColor, kStats>(g, rp, fp, rv, l, dir, bx, by, bz, cur, xs, xw, xv, out);
             return out;
         }
+    }
+    if (deferred) {
+        st->rx = rv.x;
+        st->ry = rv.y;
+        st->rz = rv.z;
+        st->l = l;
+        st->pix = (uint32_t)(i * rp.W + j);
+        st->flags = (Lp ? kRayLp : 0u) | (pre_valid ? kRayPre : 0u) | where;
+        st->pre_key = pre_key;
+        st->pre_bk = pre_bk;
+        st->pre_slot = pre_slot;
+        st->samples = out.samples;
+        st->probes = out.probes;
+        st->zt = zt;
+        st->zf = zf;
+        out.code = kRayDeferred;
     }
     return out;
 }

@@ -51,14 +51,14 @@ struct Group {
 
 // probe_run (tsdf_march.hpp) with the group: each round looks up G
 // positions at once -- lane t the one after t (first round) or t + 1 steps.
+// resumed: the lookup at rv was made (and missed) before the ray was deferred.
 template <int G>
 __device__ int gprobe_run(const GridView& g, const RayParams& rp, const Group<G>& gr, f3& rv, float& l, const f3 delta,
-                          float dl, int& steps, unsigned int& probes, float l_safe, bool pre_valid, uint32_t pre_key,
-                          uint32_t pre_bk, unsigned long long pre_slot)
+                          float dl, int& steps, unsigned int& probes, float l_safe, float l_end, bool resumed, bool pre_valid,
+                          uint32_t pre_key, uint32_t pre_bk, unsigned long long pre_slot)
 {
-    const float dmax = rp.dmax;
     int id = -1;
-    bool first = true;
+    bool first = !resumed;
     if (pre_valid) {
         const int r0 = first_slot(g, pre_key, pre_slot);
         ++probes;
@@ -67,7 +67,7 @@ __device__ int gprobe_run(const GridView& g, const RayParams& rp, const Group<G>
         if (id >= 0)
             return id;
     }
-    while (first || (id < 0 && l < dmax)) {
+    while (first || (id < 0 && l < l_end)) {
         // tile depth bounds, as in probe_run
         if (first && l < l_safe) {
             ++probes;
@@ -96,8 +96,8 @@ __device__ int gprobe_run(const GridView& g, const RayParams& rp, const Group<G>
         vb3(r, rp, x, y, z);
         const uint32_t key = prime_hash(x, y, z), bk = mix32(key) & g.mask;
         const int r0 = first_slot(g, key, g.slots[bk]);
-        // lookup k is made when every earlier one missed with l < d_max after it
-        const unsigned int m = gr.ballot(!(r0 == -1 && lr < dmax));
+        // lookup k is made when every earlier one missed with l < l_end after it
+        const unsigned int m = gr.ballot(!(r0 == -1 && lr < l_end));
         const int s = m ? __ffs(m) - 1 : G - 1;
         probes += m ? (unsigned int)(s + 1) : (unsigned int)G;
         steps += first ? s : s + 1;
@@ -227,31 +227,43 @@ __device__ RayResult march_group(const GridView& g, const Pose& pose, const RayP
     f3 n, rv0, dir;
     ray_setup(g, pose, i, j, n, rv0, dir);
     const float l_safe = (rp.use_tb && st.zt >= 0.0f) ? tb_l_safe(st.zt, n.z, dmax) : -1.0f;
+    const float l_end = (rp.use_tb && st.zf >= 0.0f) ? fminf(tb_l_far(st.zf, n.z), dmax) : dmax;
     const f3 skip = {vbl * dir.x, vbl * dir.y, vbl * dir.z};
     const f3 step = {vl * dir.x, vl * dir.y, vl * dir.z};
     f3 rv = {st.rx, st.ry, st.rz};
     float l = st.l;
-    bool Lp = (st.flags & 1u) != 0;
-    bool pre_valid = (st.flags & 2u) != 0;
+    bool Lp = (st.flags & kRayLp) != 0;
+    bool pre_valid = (st.flags & kRayPre) != 0;
+    bool in_skip = (st.flags & kRaySkip) != 0, in_advance = (st.flags & kRayAdvance) != 0;
     uint32_t pre_key = st.pre_key, pre_bk = st.pre_bk;
     unsigned long long pre_slot = st.pre_slot;
     while (l < dmax) {
-        int count = 0;
-        int id = gprobe_run<G>(g, rp, gr, rv, l, skip, vbl, count, out.probes, l_safe, pre_valid, pre_key, pre_bk,
-                               pre_slot);
-        pre_valid = false;
-        if (!(l < dmax))
-            break;
-        if (count > 0) {
-            const float back = rp.back;
-            rv.x -= back * dir.x;
-            rv.y -= back * dir.y;
-            rv.z -= back * dir.z;
-            l -= back;
+        int count = in_skip ? 1 : 0, id = -1;
+        if (!in_advance) {
+            id = gprobe_run<G>(g, rp, gr, rv, l, skip, vbl, count, out.probes, l_safe, l_end, in_skip, pre_valid,
+                               pre_key, pre_bk, pre_slot);
+            pre_valid = false;
+            if (id < 0 && l < dmax)
+                miss_to_end(l, vbl, dmax, out.probes);
+            if (!(l < dmax))
+                break;
+            if (count > 0) {
+                const float back = rp.back;
+                rv.x -= back * dir.x;
+                rv.y -= back * dir.y;
+                rv.z -= back * dir.z;
+                l -= back;
+            }
+        }
+        if (in_advance || count > 0) {
             const f3 dstep = {dt * dir.x, dt * dir.y, dt * dir.z};
             int steps = 0;
-            id = gprobe_run<G>(g, rp, gr, rv, l, dstep, dt, steps, out.probes, l_safe, false, 0u, 0u, 0ull);
+            id = gprobe_run<G>(g, rp, gr, rv, l, dstep, dt, steps, out.probes, l_safe, l_end, in_advance, false, 0u, 0u,
+                               0ull);
+            if (id < 0 && l < dmax)
+                miss_to_end(l, dt, dmax, out.probes);
         }
+        in_skip = in_advance = false;
         if (!(l < dmax))
             break;
         int bx, by, bz;

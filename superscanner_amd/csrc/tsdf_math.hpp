@@ -215,11 +215,12 @@ struct Pose {
     float pad;
 };
 
-// Pose of a render view: camera -> world rotation (row-major) and the camera
-// centre in world coordinates.
+// Pose of a render view: camera -> world rotation (row-major), the camera
+// centre in world coordinates, and world -> camera as a 3x4 row-major block.
 struct ViewPose {
     float R[9];
     float t[3];
+    float Ei[12];
 };
 
 }  // namespace tsdf
