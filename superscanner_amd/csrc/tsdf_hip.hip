@@ -1708,6 +1708,9 @@ struct tsdf_grid {
     ViewPose* view_host;  // pinned
     hipEvent_t render_done;
     bool render_staged;
+    unsigned long long* vb[2];  // least / greatest depths over the views' tiles, grown on demand
+    size_t vb_cap;              // tiles
+    uint32_t vb_epoch;
     // fixed-order reductions of the render adjoint and the tracking sums,
     // grown on demand: per-workgroup partial sums, the (voxel, value)
     // records of grad_sdf with their sorted copies, the sort's temporary
@@ -2331,6 +2334,8 @@ void tsdf_destroy(tsdf_grid* g)
     if (g->render_done)
         (void)hipEventDestroy(g->render_done);
     (void)hipFree(g->view_dev);
+    (void)hipFree(g->vb[0]);
+    (void)hipFree(g->vb[1]);
     (void)hipFree(g->red_part);
     for (int k = 0; k < 2; ++k) {
         (void)hipFree(g->rec_key[k]);
