@@ -2006,20 +2006,22 @@ void launch_raycast(tsdf_grid* g, const Pose& P, float* points, float* colors, f
     rp.use_tb = g->tune.raycast_skip == 2 && !kStats;
     // the group march replays no superblock distance field
     rp.budget = (kStats || rp.use_sb) ? 0 : g->tune.raycast_budget;
-    // How readily a ray is deferred.  One round of the 16-lane march looks up
-    // 16 positions of a ray with 16 lanes' work, the per-lane march 4 with
-    // one, so deferring pays by itself only in a wavefront with few rays left
-    // (16 lanes), and everywhere while the chip has lanes to spare.  What it
-    // has to do is bounded by the lookups of an empty march, wavefronts x
-    // d_max / vbl.  Raycast with 16 / 16, 16 / 64 and 64 / 64 lanes (run / top):
-    //   575 k  (320 x 180, 16 mm bricks)   537   541  358 us
-    //   1.2 M  (640 x 480, 40 mm)          244   226  226
-    //   2.0 M  (848 x 480, 32 mm)          206   186  185
-    //   2.25 M (640 x 360, 16 mm)          854   893 1005
-    //   9.0 M  (1280 x 720, 16 mm)        1654  1865 3389
+    // Whether rays are deferred.  One round of the 16-lane march looks up 16
+    // positions of a ray with 16 lanes' work, the per-lane march 4 with one:
+    // deferring pays while the chip has lanes to spare, and costs once it has
+    // none.  What a raycast has to do is bounded by the lookups of an empty
+    // march, wavefronts x d_max / vbl.  Raycast without and with deferral:
+    //   75 k   (160 x 120, 40 mm bricks)    269   135 us
+    //   575 k  (320 x 180, 16 mm)           571   375
+    //   1.2 M  (640 x 480, 40 mm)           275   209
+    //   2.0 M  (848 x 480, 32 mm)           180   143
+    //   2.25 M (640 x 360, 16 mm)           733  1006
+    //   3.6 M  (1280 x 720, 40 mm)          302   464
+    //   4.5 M  (1280 x 720, 32 mm)          234   272
+    //   9.0 M  (1280 x 720, 16 mm)         1319  3390
     const double lookups = (double)((rp.W + 7) / 8) * ((rp.H + 7) / 8) * (rp.dmax / rp.vbl);
-    rp.defer_run = lookups < 0.8e6 ? 64 : 16;
-    rp.defer_top = lookups < 2.1e6 ? 64 : 16;
+    if (!(lookups < 2.1e6))
+        rp.budget = 0;
     rp.lc = nullptr;  // the kernel points it at its LDS cache (TSDF_RAY_CACHE)
     const int qpar = (int)(g->ray_qepoch & 1u);
     if (rp.budget > 0)

@@ -135,8 +135,6 @@ __host__ __device__ __forceinline__ int find_brick(const GridView& g, int x, int
 // Probe result from the first slot word alone: the id, -1 (absent), or
 // kProbeMore when the slot holds another key and probing must continue.
 constexpr int kProbeMore = -2;
-// probe_run stopped at its round budget, the next lookup not yet made.
-constexpr int kProbeDeferred = -3;
 __host__ __device__ __forceinline__ int first_slot(const GridView& g, uint32_t key, unsigned long long s)
 {
     const uint32_t id = (uint32_t)s;
@@ -285,7 +283,6 @@ struct RayParams {
     int df_lo[3], df_dim[3];
     int use_tb;       // tile depth bounds replay allowed (alias certificate holds)
     int budget;       // rounds of the per-lane march before a ray is deferred (0: never)
-    int defer_run, defer_top;  // most lanes still in a probing run / in the march for a deferral there
     unsigned long long* lc;  // the workgroup's LDS cache of lookup results, or null
 };
 
@@ -587,6 +584,7 @@ enum RayFlags : uint32_t {
     kRayPre = 2u,      // pre_key, pre_bk and pre_slot hold the next lookup
     kRaySkip = 4u,     // inside the empty-block skip (steps of vbl were taken)
     kRayAdvance = 8u,  // inside the re-advance by d_trunc
+    kRayFirst = 16u,   // ... whose first lookup is still to be made
 };
 struct RayState {
     float rx, ry, rz, l;
@@ -604,7 +602,7 @@ static_assert(sizeof(RayState) == 64, "one 64-byte record per deferred ray");
 constexpr int kRayUbVoxelIndex = 1;  // TSDF_RAY_UB_VOXEL_INDEX
 constexpr int kRayUbMissingOut = 2;  // TSDF_RAY_UB_MISSING_OUT
 #ifndef TSDF_SKIP_LOOK
-#define TSDF_SKIP_LOOK 4
+#define TSDF_SKIP_LOOK 3
 #endif
 #ifndef TSDF_INNER_LOOK
 #define TSDF_INNER_LOOK 4
@@ -711,16 +709,6 @@ inline void sbdf_build_host(const uint32_t* sb_bits, const int lo[3], const int 
             }
 }
 
-// Lanes of the wavefront that run this point together (1 on the host).
-__host__ __device__ __forceinline__ int active_lanes()
-{
-#if defined(__HIP_DEVICE_COMPILE__)
-    return __popcll(__ballot(1));
-#else
-    return 1;
-#endif
-}
-
 template <bool kStats>
 __host__ __device__ __forceinline__ int probe_count(const GridView& g, const Footprint& fp, int x, int y, int z,
                                                     unsigned int& probes)
@@ -734,158 +722,6 @@ __host__ __device__ __forceinline__ int probe_count(const GridView& g, const Foo
 
 __host__ __device__ __forceinline__ f3 add3(f3 a, f3 b) { return {a.x + b.x, a.y + b.y, a.z + b.z}; }
 __host__ __device__ __forceinline__ f3 sel3(bool c, f3 a, f3 b) { return {c ? a.x : b.x, c ? a.y : b.y, c ? a.z : b.z}; }
-
-// raycastingTag for pixel (i, j), GPUVoxelGrid.cpp:561-715.
-//
-// The loops are the reference's, with two changes of schedule that keep
-// every probe, read and floating-point operation of the reference in its
-// order:
-//  - the empty-block skip (:596-604) computes its next kSkipLook positions
-//    (which depend on no memory) and issues their first hash-slot loads at
-//    once, then takes the steps in order until one hits;
-//  - the voxel walk inside a block (:638-706) likewise loads its next
-//    kInnerLook voxels at once and then applies the reference's decisions
-//    to them in order.
-// Steps are taken with selects rather than branches, so a wavefront stays
-// on one instruction stream.  Reads that lie beyond the point where the
-// reference stops are discarded.
-// One probing run of the march: the lookup at rv, then, while it misses and
-// l < dmax, steps rv += delta, l += dl, each followed by a lookup -- the
-// reference's loops at GPUVoxelGrid.cpp:589-604 (delta = vbl dir) and
-// :610-627 (delta = d_trunc dir), with two changes of schedule that keep every
-// lookup and floating-point operation in its order:
-//  - kSkipLook positions (which depend on no memory) are computed and their
-//    first hash slots loaded at once, then taken in order until one hits;
-//  - with the empty-space field (rp.use_sb), a stretch of steps whose
-//    lookups certainly miss is replayed without loading: every block within
-//    Chebyshev distance d - 1 of the block of rv is absent, and k steps (each
-//    at most vbl per axis) move the reference's block index by at most k + 3
-//    per axis, so steps 1 .. d - 4 miss.
-// Returns the brick id (>= 0) or -1; steps counts the steps taken, probes
-// every lookup of the reference (replayed ones included).  l_end <= d_max: the
-// run stops there (no brick holds a position of the ray from l_end on), and
-// the caller counts the misses up to d_max.  With a budget > 0
-// it returns kProbeDeferred once `rounds` reached it, another round would be
-// needed (every lookup so far missed, the next position not yet taken) and at
-// most rp.defer_run lanes of the wavefront are still in the run.
-//
-// pre_valid: the first slot word of the lookup at rv (key pre_key, bucket
-// pre_bk) was already loaded as pre_slot; a hit there costs no further load.
-template <bool kStats>
-__host__ __device__ __forceinline__ int probe_run(const GridView& g, const RayParams& rp, const Footprint& fp, f3& rv,
-                                                  float& l, const f3 delta, float dl, int& steps, unsigned int& probes,
-                                                  float l_safe, float l_end, int& rounds, int budget,
-                                                  bool pre_valid = false,
-                                                  uint32_t pre_key = 0, uint32_t pre_bk = 0,
-                                                  unsigned long long pre_slot = 0)
-{
-    int id = -1;
-    bool first = true;  // the lookup at rv itself has not been made
-    if (pre_valid) {
-        const int r0 = first_slot(g, pre_key, pre_slot);
-        if (kStats)
-            fp_key(fp, pre_key);
-        ++probes;
-        id = r0 == kProbeMore ? probe_from(g, pre_key, (pre_bk + 1) & g.mask) : r0;
-        cache_result(rp, pre_key, id);
-        first = false;
-        if (id >= 0)
-            return id;
-    }
-    bool have = false;  // nrep holds the replay count for the block of rv
-    int nrep = 0;
-    while (first || (id < 0 && l < l_end)) {
-        // tile depth bounds: the lookups at ray parameters below l_safe
-        // miss (l_safe <= d_max, so every such miss is followed by a step)
-        if (first && l < l_safe) {
-            ++probes;
-            first = false;
-        }
-        if (!first) {
-            for (;;) {
-                const float ln = l + dl;
-                if (!(ln < l_safe))
-                    break;
-                rv = add3(rv, delta);
-                l = ln;
-                ++steps;
-                ++probes;
-            }
-        }
-        if (rp.use_sb && !first) {
-            if (!have) {
-                int cx, cy, cz;
-                vb3(rv, rp, cx, cy, cz);
-                nrep = free_dist(rp, cx, cy, cz) - 4;
-            }
-            for (int k = 0; k < nrep && l < l_end; ++k) {
-                rv = add3(rv, delta);
-                l += dl;
-                ++steps;
-                ++probes;
-            }
-            have = false;
-            if (!(l < l_end))
-                break;
-        }
-        if (!first && budget > 0 && rounds >= budget && active_lanes() <= rp.defer_run)
-            return kProbeDeferred;
-        // positions: rv itself first (on the first round), then steps
-        uint32_t key[kSkipLook], bk[kSkipLook];
-        unsigned long long sl[kSkipLook];
-        bool cached[kSkipLook];
-        int dbl = 0, ev = 0;
-        f3 r = rv;
-#pragma unroll
-        for (int k = 0; k < kSkipLook; ++k) {
-            if (!(first && k == 0))
-                r = add3(r, delta);
-            int x, y, z;
-            vb3(r, rp, x, y, z);
-            key[k] = prime_hash(x, y, z);
-            bk[k] = mix32(key[k]) & g.mask;
-            sl[k] = lookup_slot(g, rp, key[k], bk[k], cached[k]);
-            if (k == kSkipLook - 1 && rp.use_sb) {
-                int idx;
-                dbl = df_box(rp, x, y, z, idx);
-                ev = dbl == 0 ? (int)rp.df[idx] : 0;
-            }
-        }
-        bool go = true, pend = false;
-        ++rounds;
-        uint32_t pkey = 0, pbk = 0;
-#pragma unroll
-        for (int k = 0; k < kSkipLook; ++k) {
-            const int r0 = first_slot(g, key[k], sl[k]);
-            if (!cached[k] && r0 != kProbeMore)
-                cache_result(rp, key[k], r0);
-            if (kStats && go)
-                fp_key(fp, key[k]);
-            const bool stp = go && !(first && k == 0);  // a step precedes this lookup
-            const float ln = l + dl;
-            rv = sel3(stp, add3(rv, delta), rv);
-            l = stp ? ln : l;
-            steps += stp ? 1 : 0;
-            probes += go ? 1u : 0u;
-            id = go ? r0 : id;
-            const bool more = go && r0 == kProbeMore;
-            pend = pend || more;
-            pkey = more ? key[k] : pkey;
-            pbk = more ? bk[k] : pbk;
-            go = go && r0 == -1 && l < l_end;
-        }
-        first = false;
-        if (rp.use_sb && go) {  // every lookup taken and missed: rv is the last position
-            nrep = df_dist(dbl, ev) - 4;
-            have = true;
-        }
-        if (pend) {  // first slot held another key: finish the linear probe
-            id = probe_from(g, pkey, (pbk + 1) & g.mask);
-            cache_result(rp, pkey, id);
-        }
-    }
-    return id;
-}
 
 // The rest of a probing run beyond the last brick: every lookup misses, the
 // ray ends at d_max and only the lookups are counted.
@@ -972,9 +808,45 @@ __host__ __device__ __forceinline__ void ray_setup(const GridView& g, const Pose
     rv.z -= a0 * dir.z;
 }
 
-// budget > 0: after that many probe rounds and walk windows the march stops
-// at the top of its outer loop or before the next round of a probing run,
-// returns kRayDeferred and leaves its state in *st (march_group resumes it).
+// Keeps the compiler from moving code of one wavefront across this point (no
+// instruction; nothing on the host).
+__host__ __device__ __forceinline__ void lanes_meet()
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    __builtin_amdgcn_wave_barrier();
+#endif
+}
+
+// raycastingTag for pixel (i, j), GPUVoxelGrid.cpp:561-715.
+//
+// The reference's loops: the empty-block skip (:589-604, lookups at steps of
+// vbl dir), the back-off and re-advance by d_trunc (:610-627) and the voxel
+// walk inside a block (:638-706).  Every lookup, read and floating-point
+// operation is the reference's, in its order; the schedule differs:
+//  - a round of a probing run (skip or re-advance) computes kSkipLook
+//    positions (which depend on no memory), loads their first hash slots at
+//    once and takes them in order until one hits; a round of the walk does
+//    the same with the next kInnerLook voxels.  Reads that lie beyond the
+//    point where the reference stops are discarded;
+//  - steps are taken with selects rather than branches;
+//  - the three loops are one: each pass gives every ray of a wavefront the
+//    round it is due, so a ray never waits for the others to finish the loop
+//    it has left, and a crossing is evaluated after the loop, once for all
+//    rays.  The barriers keep the compiler from undoing that;
+//  - stretches whose lookups certainly miss are replayed without loading
+//    (same positions, lengths and counts): below l_safe and from l_end on
+//    (tile depth bounds), and with the empty-space field (rp.use_sb), where
+//    every block within Chebyshev distance d - 1 of the block of rv is absent
+//    and k steps (each at most vbl per axis) move the reference's block index
+//    by at most k + 3 per axis, so steps 1 .. d - 4 miss.
+//
+// budget > 0: a ray that took that many rounds and is in no block stops: the
+// march returns kRayDeferred and leaves its state in *st (march_group resumes
+// it).
+//
+// Bound by VALU issue and the rounds of a wavefront's slowest ray.  As three
+// nested loops the same rounds took 109 us of k_raycast at 848 x 480 in the
+// room and 1 040 at 1280 x 720 over 650 k fp16 bricks.
 template <typename T, bool kColor, bool kStats>
 __host__ __device__ RayResult march(const GridView& g, const Pose& pose, const RayParams& rp, int i, int j,
                                     const Footprint& fp, float zt = -1.0f, int budget = 0, RayState* st = nullptr,
@@ -990,72 +862,158 @@ __host__ __device__ RayResult march(const GridView& g, const Pose& pose, const R
     // createNormPcdTag, GPUVoxelGrid.cpp:717-722, and the ray set-up, :565-569
     f3 n, rv, dir;
     ray_setup(g, pose, i, j, n, rv, dir);
-    // the tile bound of this ray's tile (zt < 0: no replay)
+    // the tile bounds of this ray's tile (zt, zf < 0: no replay)
     const float l_safe = (rp.use_tb && zt >= 0.0f) ? tb_l_safe(zt, n.z, dmax) : -1.0f;
     const float l_end = (rp.use_tb && zf >= 0.0f) ? fminf(tb_l_far(zf, n.z), dmax) : dmax;
     float l = 0.1f;
-    int rounds = 0;
-    const f3 skip = {vbl * dir.x, vbl * dir.y, vbl * dir.z};  // the reference's vbl * dir
-    const f3 step = {vl * dir.x, vl * dir.y, vl * dir.z};     // and vl * dir
+    const f3 step = {vl * dir.x, vl * dir.y, vl * dir.z};  // the reference's vl * dir
 
-    bool Lp = false;
+    enum { kSkip = 0, kAdvance = 1, kWalk = 2 };
+    enum { kOn = 0, kMiss, kBadIndex, kCross, kDefer };
+    int phase = kSkip, end = l < dmax ? kOn : kMiss;
+    bool first = true;     // of a run: the lookup at rv is still to be made
+    bool stepped = false;  // of a skip: steps were taken
+    bool have = false;     // nrep holds the empty-space replay count for the block of rv
+    int nrep = 0, rounds = 0;
     // the lookup at rv, loaded ahead by the voxel walk that left a block
     bool pre_valid = false;
     uint32_t pre_key = 0, pre_bk = 0;
     unsigned long long pre_slot = 0;
-    budget = st ? budget : 0;
-    uint32_t where = 0;  // kRaySkip / kRayAdvance: deferred inside that run
-    bool deferred = false;
-    while (l < dmax) {  // outer loop; done / Fn leave by return
-        if (budget > 0 && rounds >= budget && active_lanes() <= rp.defer_top) {
-            deferred = true;
-            break;
-        }
-        // ---- the block lookup at rv and the empty-block skip ------------
-        // (GPUVoxelGrid.cpp:589-604): probe rv, then steps of vbl * dir
-        int count = 0;
-        int id = probe_run<kStats>(g, rp, fp, rv, l, skip, vbl, count, out.probes, l_safe, l_end, rounds, budget,
-                                   pre_valid, pre_key, pre_bk, pre_slot);
-        pre_valid = false;
-        if (id == kProbeDeferred) {
-            where = kRaySkip;
-            deferred = true;
-            break;
-        }
-        if (id < 0 && l < dmax)
-            miss_to_end(l, vbl, dmax, out.probes);
-        if (!(l < dmax))
-            break;
-        if (count > 0) {
-            // back off and re-advance by d_trunc, GPUVoxelGrid.cpp:610-627:
-            // probe the backed-off position, then steps of d_trunc * dir
-            const float back = rp.back;
-            rv.x -= back * dir.x;
-            rv.y -= back * dir.y;
-            rv.z -= back * dir.z;
-            l -= back;
-            const f3 dstep = {dt * dir.x, dt * dir.y, dt * dir.z};
-            int steps = 0;
-            id = probe_run<kStats>(g, rp, fp, rv, l, dstep, dt, steps, out.probes, l_safe, l_end, rounds,
-                                   budget);
-            if (id == kProbeDeferred) {
-                where = kRayAdvance;
-                deferred = true;
-                break;
+    // the walk: block, brick, voxel of rv, the last sample and its weight's sign
+    int bx = 0, by = 0, bz = 0, cur = 0, vx = 0, vy = 0, vz = 0, xv = 0;
+    float xs = 0.f, xw = 0.f;
+    bool Lp = false;
+    while (end == kOn) {
+        if (phase != kWalk) {
+            const bool adv = phase == kAdvance;
+            const float dl = adv ? dt : vbl;
+            const f3 delta = {dl * dir.x, dl * dir.y, dl * dir.z};
+            int id = -1;
+            if (pre_valid) {
+                id = first_slot(g, pre_key, pre_slot);
+                if (kStats)
+                    fp_key(fp, pre_key);
+                ++out.probes;
+                if (id == kProbeMore)
+                    id = probe_from(g, pre_key, (pre_bk + 1) & g.mask);
+                cache_result(rp, pre_key, id);
+                first = false;
+                pre_valid = false;
             }
-            if (id < 0 && l < dmax)
-                miss_to_end(l, dt, dmax, out.probes);
+            if (id < 0) {
+                // the lookups at ray parameters below l_safe miss (l_safe <=
+                // d_max, so every such miss is followed by a step)
+                if (first && l < l_safe) {
+                    ++out.probes;
+                    first = false;
+                }
+                if (!first) {
+                    for (;;) {
+                        const float ln = l + dl;
+                        if (!(ln < l_safe))
+                            break;
+                        rv = add3(rv, delta);
+                        l = ln;
+                        stepped = true;
+                        ++out.probes;
+                    }
+                }
+                if (rp.use_sb && !first) {
+                    if (!have) {
+                        int cx, cy, cz;
+                        vb3(rv, rp, cx, cy, cz);
+                        nrep = free_dist(rp, cx, cy, cz) - 4;
+                    }
+                    for (int k = 0; k < nrep && l < l_end; ++k) {
+                        rv = add3(rv, delta);
+                        l += dl;
+                        stepped = true;
+                        ++out.probes;
+                    }
+                    have = false;
+                }
+                if (first || l < l_end) {
+                    // positions: rv itself first (on a run's first round), then steps
+                    uint32_t key[kSkipLook], bk[kSkipLook];
+                    unsigned long long sl[kSkipLook];
+                    bool cached[kSkipLook];
+                    int dbl = 0, ev = 0;
+                    f3 r = rv;
+#pragma unroll
+                    for (int k = 0; k < kSkipLook; ++k) {
+                        if (!(first && k == 0))
+                            r = add3(r, delta);
+                        int x, y, z;
+                        vb3(r, rp, x, y, z);
+                        key[k] = prime_hash(x, y, z);
+                        bk[k] = mix32(key[k]) & g.mask;
+                        sl[k] = lookup_slot(g, rp, key[k], bk[k], cached[k]);
+                        if (k == kSkipLook - 1 && rp.use_sb) {
+                            int idx;
+                            dbl = df_box(rp, x, y, z, idx);
+                            ev = dbl == 0 ? (int)rp.df[idx] : 0;
+                        }
+                    }
+                    bool go = true, pend = false;
+                    ++rounds;
+                    uint32_t pkey = 0, pbk = 0;
+#pragma unroll
+                    for (int k = 0; k < kSkipLook; ++k) {
+                        const int r0 = first_slot(g, key[k], sl[k]);
+                        if (!cached[k] && r0 != kProbeMore)
+                            cache_result(rp, key[k], r0);
+                        if (kStats && go)
+                            fp_key(fp, key[k]);
+                        const bool stp = go && !(first && k == 0);  // a step precedes this lookup
+                        const float ln = l + dl;
+                        rv = sel3(stp, add3(rv, delta), rv);
+                        l = stp ? ln : l;
+                        stepped = stepped || stp;
+                        out.probes += go ? 1u : 0u;
+                        id = go ? r0 : id;
+                        const bool more = go && r0 == kProbeMore;
+                        pend = pend || more;
+                        pkey = more ? key[k] : pkey;
+                        pbk = more ? bk[k] : pbk;
+                        go = go && r0 == -1 && l < l_end;
+                    }
+                    first = false;
+                    if (rp.use_sb && go) {  // every lookup taken and missed: rv is the last position
+                        nrep = df_dist(dbl, ev) - 4;
+                        have = true;
+                    }
+                    if (pend) {  // first slot held another key: finish the linear probe
+                        id = probe_from(g, pkey, (pbk + 1) & g.mask);
+                        cache_result(rp, pkey, id);
+                    }
+                }
+            }
+            if (id >= 0 || !(l < l_end)) {  // the run is over
+                if (id < 0)
+                    miss_to_end(l, dl, dmax, out.probes);
+                if (!(l < dmax)) {
+                    end = kMiss;
+                } else if (!adv && stepped) {
+                    // back off, then re-advance by d_trunc from a lookup there
+                    const float back = rp.back;
+                    rv.x -= back * dir.x;
+                    rv.y -= back * dir.y;
+                    rv.z -= back * dir.z;
+                    l -= back;
+                    phase = kAdvance;
+                    first = true;
+                    have = false;
+                } else {
+                    vb3(rv, rp, bx, by, bz);
+                    cur = id;
+                    vin3(rv, bx, by, bz, rp, vx, vy, vz);
+                    phase = kWalk;
+                }
+            }
         }
-        if (!(l < dmax))
-            break;
-        int bx, by, bz;
-        vb3(rv, rp, bx, by, bz);
-        // ---- voxel walk inside block (bx, by, bz) ----------------------
-        const int cur = id;
-        const T* brick = (const T*)g.payload + (size_t)cur * (2 * kVPB);
-        int vx, vy, vz;
-        vin3(rv, bx, by, bz, rp, vx, vy, vz);
-        while (true) {
+        lanes_meet();
+        if (phase == kWalk && end == kOn) {
+            const T* brick = (const T*)g.payload + (size_t)cur * (2 * kVPB);
             ++rounds;
             // positions r[0] = rv, r[k] = r[k - 1] + vl dir, and their
             // lengths, by the reference's additions
@@ -1120,11 +1078,8 @@ __host__ __device__ RayResult march(const GridView& g, const Pose& pose, const R
                 bool e_cached;
                 e_slot = lookup_slot(g, rp, e_key, e_bk, e_cached);
             }
-            bool stop = false;
-            int ending = 0;  // 1 left the block / range, 2 UB index, 3 Fn, 4 crossing
-            int nst = 0;     // positions taken (the march goes on from r[nst])
-            float xs = 0.f, xw = 0.f;
-            int xv = 0;
+            bool stop = false, left = false;
+            int nst = 0;  // positions taken (the march goes on from r[nst])
 #pragma unroll
             for (int k = 0; k < kInnerLook; ++k) {
                 const bool act = !stop;
@@ -1135,9 +1090,9 @@ __host__ __device__ RayResult march(const GridView& g, const Pose& pose, const R
                 if (kStats && proc)
                     fp_voxel(fp, cur, vk[k]);
                 out.samples += proc ? 1u : 0u;
-                ending = (act && vk[k] == -2) ? 1 : ending;
-                ending = (act && vk[k] == -1) ? 2 : ending;
-                ending = (proc && neg) ? (Lp ? 4 : 3) : ending;
+                left = left || (act && vk[k] == -2);
+                end = (act && vk[k] == -1) ? (int)kBadIndex : end;
+                end = (proc && neg) ? (Lp ? (int)kCross : (int)kMiss) : end;  // Fn: miss
                 xs = proc ? sk[k] : xs;
                 xw = proc ? wk[k] : xw;
                 xv = proc ? vk[k] : xv;
@@ -1150,44 +1105,41 @@ __host__ __device__ RayResult march(const GridView& g, const Pose& pose, const R
                 rv = sel3(nst == k, r[k], rv);
                 l = nst == k ? ll[k] : l;
             }
-            if (!stop) {  // walked past the window: rv = r[kInnerLook]
-                if (!in4 || !(l < dmax)) {
-                    // the inner loop test fails; rv is the window's next
-                    // position, whose lookup was loaded if it left the block
-                    pre_valid = e_found;
-                    pre_key = e_key;
-                    pre_bk = e_bk;
-                    pre_slot = e_slot;
-                    break;
-                }
-                vin3(rv, bx, by, bz, rp, vx, vy, vz);
-                continue;
-            }
-            if (ending == 1) {  // back to the outer loop from the first position that left
+            // walked past the window: rv = r[kInnerLook]; the loop test may fail there
+            left = left || (!stop && (!in4 || !(l < dmax)));
+            if (left) {
+                // back to the lookups from the first position that left,
+                // whose slot was loaded if it is in another block
                 pre_valid = e_found;
                 pre_key = e_key;
                 pre_bk = e_bk;
                 pre_slot = e_slot;
-                break;
+                phase = kSkip;
+                first = true;
+                stepped = false;
+                have = false;
+                end = l < dmax ? end : (int)kMiss;
+            } else if (end == kOn) {
+                vin3(rv, bx, by, bz, rp, vx, vy, vz);
             }
-            if (ending == 2) {
-                out.code = -kRayUbVoxelIndex;
-                return out;
-            }
-            if (ending == 3)
-                return out;  // Fn: miss
-            // zero crossing, GPUVoxelGrid.cpp:655-689
-            crossing<T, kColor, kStats>(g, rp, fp, rv, l, dir, bx, by, bz, cur, xs, xw, xv, out);
-            return out;
         }
+        lanes_meet();
+        if (budget > 0 && end == kOn && phase != kWalk && rounds >= budget && st)
+            end = kDefer;
     }
-    if (deferred) {
+    lanes_meet();
+    if (end == kCross)  // GPUVoxelGrid.cpp:655-689
+        crossing<T, kColor, kStats>(g, rp, fp, rv, l, dir, bx, by, bz, cur, xs, xw, xv, out);
+    if (end == kBadIndex)
+        out.code = -kRayUbVoxelIndex;
+    if (end == kDefer) {
         st->rx = rv.x;
         st->ry = rv.y;
         st->rz = rv.z;
         st->l = l;
         st->pix = (uint32_t)(i * rp.W + j);
-        st->flags = (Lp ? kRayLp : 0u) | (pre_valid ? kRayPre : 0u) | where;
+        st->flags = (Lp ? kRayLp : 0u) | (pre_valid ? kRayPre : 0u) |
+                    (phase == kAdvance ? kRayAdvance | (first ? kRayFirst : 0u) : (first ? 0u : kRaySkip));
         st->pre_key = pre_key;
         st->pre_bk = pre_bk;
         st->pre_slot = pre_slot;

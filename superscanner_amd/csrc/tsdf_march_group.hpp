@@ -49,7 +49,7 @@ struct Group {
     __device__ f3 from(f3 v, int k) const { return {from(v.x, k), from(v.y, k), from(v.z, k)}; }
 };
 
-// probe_run (tsdf_march.hpp) with the group: each round looks up G
+// A probing run of the march with the group: each round looks up G
 // positions at once -- lane t the one after t (first round) or t + 1 steps.
 // resumed: the lookup at rv was made (and missed) before the ray was deferred.
 template <int G>
@@ -68,7 +68,7 @@ __device__ int gprobe_run(const GridView& g, const RayParams& rp, const Group<G>
             return id;
     }
     while (first || (id < 0 && l < l_end)) {
-        // tile depth bounds, as in probe_run
+        // tile depth bounds, as in march
         if (first && l < l_safe) {
             ++probes;
             first = false;
@@ -258,7 +258,8 @@ __device__ RayResult march_group(const GridView& g, const Pose& pose, const RayP
         if (in_advance || count > 0) {
             const f3 dstep = {dt * dir.x, dt * dir.y, dt * dir.z};
             int steps = 0;
-            id = gprobe_run<G>(g, rp, gr, rv, l, dstep, dt, steps, out.probes, l_safe, l_end, in_advance, false, 0u, 0u,
+            id = gprobe_run<G>(g, rp, gr, rv, l, dstep, dt, steps, out.probes, l_safe, l_end,
+                               in_advance && !(st.flags & kRayFirst), false, 0u, 0u,
                                0ull);
             if (id < 0 && l < dmax)
                 miss_to_end(l, dt, dmax, out.probes);
