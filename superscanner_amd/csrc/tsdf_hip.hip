@@ -1721,6 +1721,8 @@ struct tsdf_grid {
     size_t rec_cap;  // records
     void* sort_tmp;
     size_t sort_tmp_cap;  // bytes
+    void* mc_buf;         // marching cubes: edge masks, bricks' shares and sums, grown on demand
+    size_t mc_cap;        // bytes
 };
 
 namespace {
@@ -2344,6 +2346,7 @@ void tsdf_destroy(tsdf_grid* g)
         (void)hipFree(g->rec_val[k]);
     }
     (void)hipFree(g->sort_tmp);
+    (void)hipFree(g->mc_buf);
     if (g->stage_host)
         (void)hipHostFree(g->stage_host);
     if (g->staging_done)

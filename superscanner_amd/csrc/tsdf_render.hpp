@@ -762,12 +762,6 @@ __global__ __launch_bounds__(kThreads) void k_track(GridView g, RenderArgs a)
     }
 }
 
-__global__ void k_fill_f64(double* p, size_t n)
-{
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
-        p[i] = 0.0;
-}
-
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
