@@ -95,11 +95,22 @@ __global__ __launch_bounds__(kThreads) void k_normals(const float* pts, int H, i
     }
 }
 
+// What tsdf_icp keeps on the device through its iterations: the transform (and
+// its float cast, as the association takes it), the best one so far, and
+// whether the iterations ended (no correspondence, or a singular sum).
+struct IcpState {
+    double T[16], best[16];
+    float Tf[12];
+    float lowest, best_fit;
+    int stop;
+};
+
 struct IcpArgs {
     const float* x;
     const float* y;
     const float* yn;
     float T[12];  // Txy, 3x4 row-major
+    const IcpState* it;  // or the iterations' own (then T is not read)
     Camera cam;
     int H, W;
     int n_search;
@@ -126,22 +137,97 @@ constexpr int kIcpTile = 16;
 constexpr int kIcpLds = TSDF_ICP_LDS;  // staged candidates per workgroup
 constexpr int kIcpLdsAlloc = kIcpLds > 0 ? kIcpLds : 1;
 
-// candidate (r, c): from the staged box (origin r0, c0, width bw) or global memory
-template <bool kLds>
-__device__ __forceinline__ f3 icp_cand(const float* lx, const float* ly, const float* lz, int r, int c, int r0,
-                                      int c0, int bw, const float* g, unsigned int q)
+// The scan of a window in the staged box (origin r0, c0, width bw).  A
+// candidate that cannot qualify (z == 0, or n.x == 0 for point to plane) is
+// staged with x = NaN: its distance compares false.
+//
+// Point to point selects by dist = sqrt(sq) < the least dist so far (at first
+// max_dist), strictly, in scan order.  The squared lengths decide without the
+// root: with s the least one's (at first max_dist^2, rounded up by a few ulp),
+// sq < s (1 - 2^-20) gives a smaller root for certain (a relative 2^-21 below,
+// several ulp) and sq >= s none; only between the two are the roots taken.
+// The caller has checked 1e-9 <= max_dist.
+//
+// 12 VALU instructions and one LDS read a candidate (two candidates at a time:
+// a window is 2 n wide); bound by issuing them and by the staging's latency.
+// n = 5: 38.1 -> 22.1 us point to point at 640 x 480, 57.3 -> 29.5 us point to
+// plane at 848 x 480, with the root in the loop, the best point carried along
+// and three reads a candidate before.
+template <bool kPlane>
+__device__ __forceinline__ f3 icp_scan_lds(const IcpArgs& a, f3 px, int ci, int cj, const float4* ly, const float2* ln,
+                                           int r0, int c0, int bw)
 {
-    if (kLds) {
-        const int o = (r - r0) * bw + (c - c0);
-        return f3{lx[o], ly[o], lz[o]};
+    const int ns = a.n_search;
+    int best = -1;
+    if (!kPlane) {
+        const float least0 = fminf(a.max_dist, 1e6f);
+        const float s0 = least0 * least0 * (1.0f + 0x1p-20f);  // at or above its square
+        float s = s0;
+        float sure = s0 * (1.0f - 0x1p-18f);  // below its square for certain
+        for (int r = ci - ns; r < ci + ns; ++r) {
+            const int row = (r - r0) * bw - c0;
+            for (int c = cj - ns; c < cj + ns; c += 2) {
+                const float4 y[2] = {ly[row + c], ly[row + c + 1]};
+                const int best_was = best;
+                const float s_was = s, sure_was = sure;
+                bool near = false;  // one that only the roots can tell from the best
+                float sq[2];
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    const f3 dv = sub3(f3{y[k].x, y[k].y, y[k].z}, px);
+                    sq[k] = dv.x * dv.x + dv.y * dv.y + dv.z * dv.z;
+                    const bool take = sq[k] < sure;
+                    near = near || (sq[k] < s && !take);
+                    best = take ? row + c + k : best;
+                    s = take ? sq[k] : s;
+                    sure = take ? sq[k] * (1.0f - 0x1p-20f) - 1e-30f : sure;  // (less is safe: denormals)
+                }
+                if (__builtin_expect(near, 0)) {
+                    best = best_was;
+                    s = s_was;
+                    sure = sure_was;
+                    for (int k = 0; k < 2; ++k)
+                        if (sqrtf(sq[k]) < (best < 0 ? least0 : sqrtf(s))) {
+                            best = row + c + k;
+                            s = sq[k];
+                            sure = sq[k] * (1.0f - 0x1p-20f) - 1e-30f;
+                        }
+                }
+            }
+        }
+        if (best < 0)
+            return f3{0.0f, 0.0f, 0.0f};
+        const float4 y = ly[best];
+        return f3{y.x, y.y, y.z};
     }
-    return ld3(g, q);
+    float least = fminf(a.max_dist, 1e6f);
+    float bd = 0.0f;
+    for (int r = ci - ns; r < ci + ns; ++r) {
+        const int row = (r - r0) * bw - c0;
+        for (int c = cj - ns; c < cj + ns; c += 2) {
+            const float4 y[2] = {ly[row + c], ly[row + c + 1]};
+            const float2 n2[2] = {ln[row + c], ln[row + c + 1]};
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                const f3 dv = sub3(f3{y[k].x, y[k].y, y[k].z}, px);
+                const float d = dv.x * y[k].w + dv.y * n2[k].x + dv.z * n2[k].y;
+                const bool take = fabsf(d) < least;
+                best = take ? row + c + k : best;
+                bd = take ? d : bd;
+                least = take ? fabsf(d) : least;
+            }
+        }
+    }
+    if (best < 0)
+        return f3{0.0f, 0.0f, 0.0f};
+    const float nx = ly[best].w;
+    const float2 n2 = ln[best];
+    return f3{px.x + bd * nx, px.y + bd * n2.x, px.z + bd * n2.y};
 }
 
-template <bool kLds, bool kPlane>
-__device__ __forceinline__ f3 icp_scan(const IcpArgs& a, f3 px, int ci, int cj, const float* ly_x, const float* ly_y,
-                                       const float* ly_z, const float* ln_x, const float* ln_y, const float* ln_z,
-                                       int r0, int c0, int bw)
+// The same from global memory, for a tile whose windows spread too far.
+template <bool kPlane>
+__device__ __forceinline__ f3 icp_scan(const IcpArgs& a, f3 px, int ci, int cj)
 {
     f3 best{0.0f, 0.0f, 0.0f};
     const int ns = a.n_search;
@@ -153,7 +239,7 @@ __device__ __forceinline__ f3 icp_scan(const IcpArgs& a, f3 px, int ci, int cj, 
     for (int r = ci - ns; r < ci + ns; ++r) {
         for (int c = cj - ns; c < cj + ns; ++c) {
             const unsigned int q = (unsigned int)(r * a.W + c);
-            const f3 py = icp_cand<kLds>(ly_x, ly_y, ly_z, r, c, r0, c0, bw, a.y, q);
+            const f3 py = ld3(a.y, q);
             if (!kPlane) {
                 const f3 dv = sub3(py, px);
                 const float sq = dv.x * dv.x + dv.y * dv.y + dv.z * dv.z;
@@ -166,7 +252,7 @@ __device__ __forceinline__ f3 icp_scan(const IcpArgs& a, f3 px, int ci, int cj, 
                     }
                 }
             } else {
-                const f3 nv = icp_cand<kLds>(ln_x, ln_y, ln_z, r, c, r0, c0, bw, a.yn, q);
+                const f3 nv = ld3(a.yn, q);
                 if (py.z != 0.0f && nv.x != 0.0f) {
                     const f3 dv = sub3(py, px);
                     const float d = dv.x * nv.x + dv.y * nv.y + dv.z * nv.z;
@@ -185,9 +271,16 @@ __device__ __forceinline__ f3 icp_scan(const IcpArgs& a, f3 px, int ci, int cj, 
 template <bool kPlane>
 __global__ __launch_bounds__(kIcpTile * kIcpTile) void k_icp_associate(IcpArgs a)
 {
-    __shared__ float sy[3][kIcpLdsAlloc];
-    __shared__ float sn[kPlane ? 3 : 1][kPlane ? kIcpLdsAlloc : 1];
+    __shared__ float4 sy[kIcpLdsAlloc];                  // y, and n.x for point to plane
+    __shared__ float2 sn[kPlane ? kIcpLdsAlloc : 1];     // n.y, n.z
     __shared__ int box[4];  // row min, row max (exclusive), col min, col max (exclusive)
+    if (a.it) {
+        if (a.it->stop)
+            return;
+#pragma unroll
+        for (int k = 0; k < 12; ++k)
+            a.T[k] = a.it->Tf[k];
+    }
     const int tiles_x = (a.W + kIcpTile - 1) / kIcpTile;
     const int i = (int)(blockIdx.x / tiles_x) * kIcpTile + (int)(threadIdx.x / kIcpTile);
     const int j = (int)(blockIdx.x % tiles_x) * kIcpTile + (int)(threadIdx.x % kIcpTile);
@@ -217,12 +310,21 @@ __global__ __launch_bounds__(kIcpTile * kIcpTile) void k_icp_associate(IcpArgs a
             box[2] = 0x7FFFFFFF;
             box[3] = (int)0x80000000u;
         }
+        // the wavefront's box, then one set of atomics per wavefront
+        int b0 = act ? ci - ns : 0x7FFFFFFF, b1 = act ? ci + ns : (int)0x80000000u;
+        int b2 = act ? cj - ns : 0x7FFFFFFF, b3 = act ? cj + ns : (int)0x80000000u;
+        for (int o = 32; o > 0; o >>= 1) {
+            b0 = min(b0, __shfl_xor(b0, o));
+            b1 = max(b1, __shfl_xor(b1, o));
+            b2 = min(b2, __shfl_xor(b2, o));
+            b3 = max(b3, __shfl_xor(b3, o));
+        }
         __syncthreads();
-        if (act) {
-            atomicMin(&box[0], ci - ns);
-            atomicMax(&box[1], ci + ns);
-            atomicMin(&box[2], cj - ns);
-            atomicMax(&box[3], cj + ns);
+        if ((threadIdx.x & 63) == 0) {
+            atomicMin(&box[0], b0);
+            atomicMax(&box[1], b1);
+            atomicMin(&box[2], b2);
+            atomicMax(&box[3], b3);
         }
         __syncthreads();
         // a workgroup without an active pixel leaves the sentinels in place:
@@ -234,34 +336,29 @@ __global__ __launch_bounds__(kIcpTile * kIcpTile) void k_icp_associate(IcpArgs a
         c0 = any ? box[2] : 0;
         const int bh = any ? box[1] - box[0] : 0;
         bw = any ? box[3] - box[2] : 0;
-        stage = any && bh * bw <= kIcpLds;
+        stage = any && bh <= kIcpLds && bh * bw <= kIcpLds && a.max_dist >= 1e-9f;
         if (stage) {
             for (int t = threadIdx.x; t < bh * bw; t += kIcpTile * kIcpTile) {
                 const int r = r0 + t / bw, c = c0 + t % bw;
                 const unsigned int q = (unsigned int)(r * a.W + c);
                 const f3 v = ld3(a.y, q);
-                sy[0][t] = v.x;
-                sy[1][t] = v.y;
-                sy[2][t] = v.z;
+                bool ok = v.z != 0.0f;
+                float4 s = make_float4(v.x, v.y, v.z, 0.0f);
                 if (kPlane) {
                     const f3 nv = ld3(a.yn, q);
-                    sn[0][t] = nv.x;
-                    sn[kPlane ? 1 : 0][t] = nv.y;
-                    sn[kPlane ? 2 : 0][t] = nv.z;
+                    ok = ok && nv.x != 0.0f;
+                    s.w = nv.x;
+                    sn[t] = make_float2(nv.y, nv.z);
                 }
+                s.x = ok ? s.x : __builtin_nanf("");  // never selected
+                sy[t] = s;
             }
         }
         __syncthreads();
     }
     f3 best{0.0f, 0.0f, 0.0f};
-    if (act) {
-        if (stage)
-            best = icp_scan<true, kPlane>(a, px, ci, cj, sy[0], sy[1], sy[2], sn[0], sn[kPlane ? 1 : 0],
-                                          sn[kPlane ? 2 : 0], r0, c0, bw);
-        else
-            best = icp_scan<false, kPlane>(a, px, ci, cj, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0,
-                                           0);
-    }
+    if (act)
+        best = stage ? icp_scan_lds<kPlane>(a, px, ci, cj, sy, sn, r0, c0, bw) : icp_scan<kPlane>(a, px, ci, cj);
     if (in)
         st3(a.out, k, best);
 }
@@ -273,6 +370,7 @@ struct MomentArgs {
     const float* x;
     const float* xn;
     double T[12];
+    const IcpState* it;  // or the iterations' own (then T is not read)
     unsigned int n;
     double* partial;  // [kIcpBlocks][kIcpMoments]
 };
@@ -286,6 +384,13 @@ __device__ __forceinline__ double wave_sum_f64(double v)
 
 __global__ __launch_bounds__(kThreads) void k_icp_moments(MomentArgs a)
 {
+    if (a.it) {
+        if (a.it->stop)
+            return;
+#pragma unroll
+        for (int k = 0; k < 12; ++k)
+            a.T[k] = a.it->T[k];
+    }
     double m[kIcpMoments];
 #pragma unroll
     for (int q = 0; q < kIcpMoments; ++q)
@@ -351,11 +456,82 @@ __global__ __launch_bounds__(kIcpFinalThreads) void k_icp_moments_final(const do
     }
 }
 
+// polar3 and the rest of an iteration, kokkosICP.cpp:117-185, in double: the
+// centroids, the rotation and the transform, which is kept as the best one
+// when this iteration's RMSE is the lowest.
+__host__ __device__ bool polar3(const double* A, double* Q);
+
+// The blocks' partial sums of an iteration, added as k_icp_moments_final adds
+// them, then the iteration's step by one thread: the transform stays on the
+// device, so the iterations follow each other without the host.  12 us, the
+// polar iteration's divisions one after the other; with the host in every
+// iteration (a copy back, a wait, the launches) an iteration took 70 us at
+// 640 x 480, without 46.
+constexpr int kIcpStepThreads = 1024;
+
+__global__ __launch_bounds__(kIcpStepThreads) void k_icp_step(const double* partial, int n_blocks, IcpState* st)
+{
+    __shared__ double m[kIcpMoments];
+    if (st->stop)
+        return;
+    const int lane = threadIdx.x & 63;
+    for (int q = threadIdx.x >> 6; q < kIcpMoments; q += kIcpStepThreads / 64) {
+        double s = 0.0;
+        for (int b = lane; b < n_blocks; b += 64)
+            s += partial[(size_t)b * kIcpMoments + q];
+        s = wave_sum_f64(s);
+        if (lane == 0)
+            m[q] = s;
+    }
+    __syncthreads();
+    if (threadIdx.x != 0)
+        return;
+    if (m[1] == 0.0) {  // no correspondence: the reference's sums turn to NaN and nothing improves
+        st->stop = 1;
+        return;
+    }
+    const double nc = m[1];
+    const double cx[3] = {m[2] / nc, m[3] / nc, m[4] / nc}, cy[3] = {m[5] / nc, m[6] / nc, m[7] / nc};
+    const float rmse = sqrtf((float)(m[17] / nc));
+    const float fit = (float)(nc / m[0]);
+    if (fit > st->best_fit)
+        st->best_fit = fit;
+    // H = sum (x - cx)(y - cy)^T = sum x y^T - n cx cy^T; the rotation is
+    // the polar factor of H^T
+    double Ht[9];
+    for (int a = 0; a < 3; ++a)
+        for (int b = 0; b < 3; ++b)
+            Ht[3 * b + a] = m[8 + 3 * a + b] - nc * cx[a] * cy[b];
+    double R[9];
+    if (!polar3(Ht, R)) {
+        st->stop = 1;
+        return;
+    }
+    double T[16];
+    for (int a = 0; a < 3; ++a) {
+        for (int b = 0; b < 3; ++b)
+            T[4 * a + b] = R[3 * a + b];
+        T[4 * a + 3] = cy[a] - (R[3 * a] * cx[0] + R[3 * a + 1] * cx[1] + R[3 * a + 2] * cx[2]);
+    }
+    T[12] = T[13] = T[14] = 0.0;
+    T[15] = 1.0;
+    for (int k = 0; k < 16; ++k)
+        st->T[k] = T[k];
+    for (int k = 0; k < 12; ++k)
+        st->Tf[k] = (float)T[k];
+    if (rmse < st->lowest) {
+        st->lowest = rmse;
+        for (int k = 0; k < 16; ++k)
+            st->best[k] = T[k];
+    }
+}
+
 // The sums into buf + kIcpBlocks * kIcpMoments (device), with buf's first
 // kIcpBlocks * kIcpMoments doubles as the partial sums.
 void launch_icp_moments(const float* x, const float* xn, const double* T16, unsigned int n, double* buf, hipStream_t s)
 {
     MomentArgs a;
+    a.it = nullptr;
     a.x = x;
     a.xn = xn;
     for (int k = 0; k < 12; ++k)
@@ -406,7 +582,8 @@ struct IcpWorkspace {
     size_t n_cap = 0;  // pixels the point maps hold
     float* buf = nullptr;
     double* mom = nullptr;
-    double* mom_host = nullptr;
+    IcpState* state = nullptr;
+    IcpState* state_host = nullptr;  // pinned
 };
 constexpr int kIcpMaxDevices = 64;
 IcpWorkspace g_icp_ws[kIcpMaxDevices];
@@ -418,8 +595,12 @@ bool icp_workspace(IcpWorkspace& w, size_t n)
         w.mom = nullptr;
         return false;
     }
-    if (!w.mom_host && hipHostMalloc(&w.mom_host, kIcpMoments * sizeof(double), hipHostMallocDefault) != hipSuccess) {
-        w.mom_host = nullptr;
+    if (!w.state && hipMalloc(&w.state, sizeof(IcpState)) != hipSuccess) {
+        w.state = nullptr;
+        return false;
+    }
+    if (!w.state_host && hipHostMalloc(&w.state_host, sizeof(IcpState), hipHostMallocDefault) != hipSuccess) {
+        w.state_host = nullptr;
         return false;
     }
     if (n > w.n_cap) {
@@ -506,7 +687,7 @@ void mat4_mul(const double* a, const double* b, double* o)
 // 1986).  With A = H^T and H = U S V^T this is V U^T, the rotation of the
 // SVD step of the reference (kokkosICP.cpp:173-177).  False when A is
 // singular or the iteration does not settle.
-bool polar3(const double* A, double* Q)
+__host__ __device__ bool polar3(const double* A, double* Q)
 {
     double X[9];
     for (int k = 0; k < 9; ++k)
@@ -516,7 +697,7 @@ bool polar3(const double* A, double* Q)
         const double c10 = X[2] * X[7] - X[1] * X[8], c11 = X[0] * X[8] - X[2] * X[6], c12 = X[1] * X[6] - X[0] * X[7];
         const double c20 = X[1] * X[5] - X[2] * X[4], c21 = X[2] * X[3] - X[0] * X[5], c22 = X[0] * X[4] - X[1] * X[3];
         const double det = X[0] * c00 + X[1] * c01 + X[2] * c02;
-        if (!(det != 0.0) || !std::isfinite(det))
+        if (!(det != 0.0) || !isfinite(det))
             return false;
         // X^-T = cofactor matrix / det
         const double it_[9] = {c00 / det, c01 / det, c02 / det, c10 / det, c11 / det,
@@ -526,7 +707,7 @@ bool polar3(const double* A, double* Q)
             nx += X[k] * X[k];
             ni += it_[k] * it_[k];
         }
-        const double g = std::sqrt(std::sqrt(ni / nx));
+        const double g = sqrt(sqrt(ni / nx));
         double diff = 0.0;
         for (int k = 0; k < 9; ++k) {
             const double v = 0.5 * (g * X[k] + it_[k] / g);
@@ -578,6 +759,42 @@ tsdf_status tsdf_points_to_normals(const float* points, int32_t height, int32_t 
     return TSDF_OK;
 }
 
+}  // extern "C"
+
+namespace {
+
+// The association with Txy, or with the iterations' own transform.
+tsdf_status launch_associate(const float* x_points, const float* y_points, const float* y_normals, const float* Txy,
+                             const IcpState* it, const tsdf_view* cam, const tsdf_icp_params* p, float* x_nearest,
+                             void* stream)
+{
+    IcpArgs a;
+    a.x = x_points;
+    a.y = y_points;
+    a.yn = y_normals;
+    for (int k = 0; k < 12; ++k)
+        a.T[k] = Txy ? Txy[k] : 0.0f;
+    a.cam = icp_camera(cam);
+    a.H = cam->height;
+    a.W = cam->width;
+    a.n_search = p->n_search;
+    a.max_dist = p->max_dist;
+    a.type = p->type;
+    a.out = x_nearest;
+    a.it = it;
+    const int tiles = ((a.W + kIcpTile - 1) / kIcpTile) * ((a.H + kIcpTile - 1) / kIcpTile);
+    if (a.type == TSDF_ICP_POINT_TO_PLANE)
+        hipLaunchKernelGGL(k_icp_associate<true>, dim3(tiles), dim3(kIcpTile * kIcpTile), 0, (hipStream_t)stream, a);
+    else
+        hipLaunchKernelGGL(k_icp_associate<false>, dim3(tiles), dim3(kIcpTile * kIcpTile), 0, (hipStream_t)stream, a);
+    HIPC(hipGetLastError());
+    return TSDF_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
 tsdf_status tsdf_icp_associate(const float* x_points, const float* y_points, const float* y_normals,
                                const float Txy[16], const tsdf_view* cam, const tsdf_icp_params* p, float* x_nearest,
                                void* stream)
@@ -586,26 +803,7 @@ tsdf_status tsdf_icp_associate(const float* x_points, const float* y_points, con
         return fail(TSDF_BAD_ARG, "NULL buffer, bad view or bad parameters");
     if (p->type == TSDF_ICP_POINT_TO_PLANE && !y_normals)
         return fail(TSDF_BAD_ARG, "point-to-plane association needs the normals of y");
-    IcpArgs a;
-    a.x = x_points;
-    a.y = y_points;
-    a.yn = y_normals;
-    for (int k = 0; k < 12; ++k)
-        a.T[k] = Txy[k];
-    a.cam = icp_camera(cam);
-    a.H = cam->height;
-    a.W = cam->width;
-    a.n_search = p->n_search;
-    a.max_dist = p->max_dist;
-    a.type = p->type;
-    a.out = x_nearest;
-    const int tiles = ((a.W + kIcpTile - 1) / kIcpTile) * ((a.H + kIcpTile - 1) / kIcpTile);
-    if (a.type == TSDF_ICP_POINT_TO_PLANE)
-        hipLaunchKernelGGL(k_icp_associate<true>, dim3(tiles), dim3(kIcpTile * kIcpTile), 0, (hipStream_t)stream, a);
-    else
-        hipLaunchKernelGGL(k_icp_associate<false>, dim3(tiles), dim3(kIcpTile * kIcpTile), 0, (hipStream_t)stream, a);
-    HIPC(hipGetLastError());
-    return TSDF_OK;
+    return launch_associate(x_points, y_points, y_normals, Txy, nullptr, cam, p, x_nearest, stream);
 }
 
 tsdf_status tsdf_icp_moments(const float* x_points, const float* x_nearest, const double Txy[16], int32_t height,
@@ -679,11 +877,13 @@ tsdf_status tsdf_icp_release(void)
     // finished call still uses the buffers
     (void)hipFree(ws.buf);
     (void)hipFree(ws.mom);
-    if (ws.mom_host)
-        (void)hipHostFree(ws.mom_host);
+    (void)hipFree(ws.state);
+    if (ws.state_host)
+        (void)hipHostFree(ws.state_host);
     ws.buf = nullptr;
     ws.mom = nullptr;
-    ws.mom_host = nullptr;
+    ws.state = nullptr;
+    ws.state_host = nullptr;
     ws.n_cap = 0;
     return TSDF_OK;
 }
@@ -717,63 +917,48 @@ tsdf_status tsdf_icp(const uint16_t* depth1, const uint16_t* depth2, const doubl
     if (!icp_workspace(ws, n))
         return fail(TSDF_HIP_ERROR, "icp workspace allocation failed");
     float* buf = ws.buf;
-    double* mom = ws.mom;
-    double* mom_host = ws.mom_host;
+    IcpState& st = *ws.state_host;
     float *x = buf, *y = buf + 3 * n, *yn = buf + 6 * n, *xn = buf + 9 * n;
     tsdf_status r = tsdf_depth_to_points(depth1, cam, x, stream);
     if (r == TSDF_OK)
         r = tsdf_depth_to_points(depth2, cam, y, stream);
     if (r == TSDF_OK)
         r = tsdf_points_to_normals(y, cam->height, cam->width, yn, stream);
-    float lowest = 1e6f, best_fit = 0.0f;
-    double best[16] = {1, 0, 0, 0, 0, 1, 0, 0, 0, 0, 1, 0, 0, 0, 0, 1};
+    memset(&st, 0, sizeof(st));
+    for (int k = 0; k < 16; ++k) {
+        st.T[k] = T[k];
+        st.best[k] = k % 5 == 0 ? 1.0 : 0.0;
+    }
+    for (int k = 0; k < 12; ++k)
+        st.Tf[k] = (float)T[k];
+    st.lowest = 1e6f;
+    auto hip = [&](hipError_t e) {
+        if (e != hipSuccess && r == TSDF_OK)
+            r = fail(TSDF_HIP_ERROR, std::string("icp: ") + hipGetErrorString(e));
+    };
+    if (r == TSDF_OK)
+        hip(hipMemcpyAsync(ws.state, &st, sizeof(st), hipMemcpyHostToDevice, s));
+    MomentArgs ma;
+    memset(&ma, 0, sizeof(ma));
+    ma.x = x;
+    ma.xn = xn;
+    ma.it = ws.state;
+    ma.n = (unsigned int)n;
+    ma.partial = ws.mom;
     for (int it = 0; it < p->n_iterations && r == TSDF_OK; ++it) {
-        float Tf[16];
-        for (int k = 0; k < 16; ++k)
-            Tf[k] = (float)T[k];
-        r = tsdf_icp_associate(x, y, yn, Tf, cam, p, xn, stream);
-        if (r == TSDF_OK) {
-            launch_icp_moments(x, xn, T, (unsigned int)n, mom, s);
-            hipError_t e = hipGetLastError();
-            if (e == hipSuccess)
-                e = hipMemcpyAsync(mom_host, mom + (size_t)kIcpBlocks * kIcpMoments, kIcpMoments * sizeof(double),
-                                   hipMemcpyDeviceToHost, s);
-            if (e == hipSuccess)
-                e = hipStreamSynchronize(s);
-            if (e != hipSuccess)
-                r = fail(TSDF_HIP_ERROR, std::string("icp moments: ") + hipGetErrorString(e));
-        }
-        const double* m = mom_host;
-        if (r != TSDF_OK || m[1] == 0.0)
-            break;  // no correspondence: the reference's sums turn to NaN and nothing improves
-        const double nc = m[1];
-        const double cx[3] = {m[2] / nc, m[3] / nc, m[4] / nc}, cy[3] = {m[5] / nc, m[6] / nc, m[7] / nc};
-        const float rmse = std::sqrt((float)(m[17] / nc));
-        const float fit = (float)(nc / m[0]);
-        if (fit > best_fit)
-            best_fit = fit;
-        // H = sum (x - cx)(y - cy)^T = sum x y^T - n cx cy^T; the rotation is
-        // the polar factor of H^T
-        double Ht[9];
-        for (int a = 0; a < 3; ++a)
-            for (int b = 0; b < 3; ++b)
-                Ht[3 * b + a] = m[8 + 3 * a + b] - nc * cx[a] * cy[b];
-        double R[9];
-        if (!polar3(Ht, R))
-            break;
-        for (int a = 0; a < 3; ++a) {
-            for (int b = 0; b < 3; ++b)
-                T[4 * a + b] = R[3 * a + b];
-            T[4 * a + 3] = cy[a] - (R[3 * a] * cx[0] + R[3 * a + 1] * cx[1] + R[3 * a + 2] * cx[2]);
-        }
-        T[12] = T[13] = T[14] = 0.0;
-        T[15] = 1.0;
-        if (rmse < lowest) {
-            lowest = rmse;
-            for (int k = 0; k < 16; ++k)
-                best[k] = T[k];
+        r = launch_associate(x, y, yn, nullptr, ws.state, cam, p, xn, stream);
+        hipLaunchKernelGGL(k_icp_moments, dim3(kIcpBlocks), dim3(kThreads), 0, s, ma);
+        hipLaunchKernelGGL(k_icp_step, dim3(1), dim3(kIcpStepThreads), 0, s, ws.mom, kIcpBlocks, ws.state);
+        hip(hipGetLastError());
+        if (it % 64 == 63 && r == TSDF_OK) {  // many iterations: see whether they ended
+            hip(hipMemcpyAsync(&st, ws.state, sizeof(st), hipMemcpyDeviceToHost, s));
+            hip(hipStreamSynchronize(s));
+            if (st.stop)
+                break;
         }
     }
+    if (r == TSDF_OK)
+        hip(hipMemcpyAsync(&st, ws.state, sizeof(st), hipMemcpyDeviceToHost, s));
     if (r != TSDF_OK)
         return r;
     // the launches of an n_iterations == 0 call end here too
@@ -781,11 +966,11 @@ tsdf_status tsdf_icp(const uint16_t* depth1, const uint16_t* depth2, const doubl
     if (se != hipSuccess)
         return fail(TSDF_HIP_ERROR, std::string("icp: ") + hipGetErrorString(se));
     for (int k = 0; k < 16; ++k)
-        T_out[k] = best[k];
+        T_out[k] = st.best[k];
     if (rmse_out)
-        *rmse_out = lowest;
+        *rmse_out = st.lowest;
     if (fitness_out)
-        *fitness_out = best_fit;
+        *fitness_out = st.best_fit;
     return TSDF_OK;
 }
 
