@@ -653,7 +653,7 @@ def fp16_scale_leg(dev, frames):
 
 
 CAL_BYTES = 256 << 20   # calibration copy: 256 MiB read + 256 MiB written
-KERNEL_NAMES = {"collect": "k_collect(", "integrate": "k_integrate<", "ray_bounds": "k_ray_bounds<",
+KERNEL_NAMES = {"collect": "k_collect<", "integrate": "k_integrate<", "ray_bounds": "k_ray_bounds<",
                 "ray_march": "k_raycast<", "ray_tail": "k_raycast_tail<"}
 RAYCAST_PARTS = ("ray_bounds", "ray_march", "ray_tail")  # the kernels of one tsdf_raycast
 

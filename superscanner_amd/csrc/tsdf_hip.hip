@@ -69,8 +69,20 @@ struct Offsets {
 };
 
 constexpr int kThreads = 256;
+// Collection tiles (pixels of a workgroup, in 8 x 8 patches) and their block
+// sets.  A set holds kLdsSet blocks; a full one falls back to claiming blocks
+// one by one, which costs far more than the set.  Large images take 32 x 8
+// pixels, a patch per wavefront; images of at most kSmallPatches patches a CU
+// take one patch a workgroup: fewer workgroups than that leave the chip idle,
+// and the patches of a small image are wide, with hundreds of blocks each.
+// Collection, 64 x 8 / 32 x 8 / 16 x 16 / 8 x 8 pixels a tile:
+//   160 x 120 (300 patches, 5 mm voxels)      75    31    25    14 us
+//   320 x 180 (920, 2 mm)                    112    62    62    28
+//   320 x 240 (1 200, 5 mm)                   34    17    16    18
+//   848 x 480 (6 360, 4 mm)                   27    25    25    44
+//   1280 x 720 (14 400, 2 mm)                 95    54    56   130
 #ifndef TSDF_TILE_W
-#define TSDF_TILE_W 64
+#define TSDF_TILE_W 32
 #endif
 #ifndef TSDF_TILE_H
 #define TSDF_TILE_H 8
@@ -78,16 +90,14 @@ constexpr int kThreads = 256;
 #ifndef TSDF_LDS_SET
 #define TSDF_LDS_SET 1024
 #endif
-// Collection tile: 64 x 8 pixels = 8 patches of 8 x 8, two per wavefront.
-// Its block set holds kLdsSet blocks (8 KiB); a tile sees several tens of
-// blocks on average, but grazing views put hundreds in one tile, and a full
-// set falls back to claiming blocks one by one, which costs far more than
-// the set.
 constexpr int kTileW = TSDF_TILE_W;
 constexpr int kTileH = TSDF_TILE_H;
 constexpr int kLdsSet = TSDF_LDS_SET;
+constexpr int kSmallPatches = 4;
 // A batch pass collects several ops at once (grid.z = op), which fills the
 // GPU with larger tiles; larger tiles also see a block fewer times per op.
+// 8 ops, 64 x 16 / 16 x 16 pixels: 848 x 480 89 / 104 us, 424 x 240 47 / 44,
+// 160 x 120 173 / 31.
 #ifndef TSDF_BATCH_TILE_W
 #define TSDF_BATCH_TILE_W 64
 #endif
@@ -96,7 +106,7 @@ constexpr int kLdsSet = TSDF_LDS_SET;
 #endif
 constexpr int kBatchTileW = TSDF_BATCH_TILE_W;
 constexpr int kBatchTileH = TSDF_BATCH_TILE_H;
-constexpr int kBatchLdsSet = 2048;  // four times the plain tile's pixels
+constexpr int kBatchLdsSet = 2048;
 constexpr int kMaxOps = 256;    // ops per batched pass
 constexpr int kMaskWords = kMaxOps / 32;
 
@@ -332,7 +342,7 @@ __global__ void k_reset(GridView g, uint32_t* op_mask, size_t op_mask_words)
 // ---------------------------------------------------------------------------
 // k_collect: block allocation (vbCollectionTag, GPUVoxelGrid.cpp:471-514)
 // ---------------------------------------------------------------------------
-// One workgroup per kTileW x kTileH pixel tile.  Each valid pixel enumerates the
+// One workgroup per kTW x kTH pixel tile.  Each valid pixel enumerates the
 // blocks of its +-trunc box into an LDS set, so the global table sees each
 // block once per tile; then the tile's set is claimed against the global
 // table with wavefront-aggregated appends to the touched list.  The pixel's
@@ -508,20 +518,21 @@ __device__ void collect_tile(const GridView& g, const OpDesc& op, uint32_t epoch
         g.touched[app_base + e] = app[e];
 }
 
+template <int kTW, int kTH>
 __global__ __launch_bounds__(kThreads) void k_collect(GridView g, OpDesc op, uint32_t epoch, int par)
 {
-    collect_tile<false, kTileW, kTileH, kLdsSet>(g, op, epoch, par, nullptr, 0);
+    collect_tile<false, kTW, kTH, kLdsSet>(g, op, epoch, par, nullptr, 0);
 }
 
 // A batch pass reads its call stamp from device memory (*epoch_base + pass)
 // so that a captured graph of the whole batch can be replayed with new
 // stamps.
+template <int kTW, int kTH>
 __global__ __launch_bounds__(kThreads) void k_collect_batch(GridView g, const OpDesc* ops,
                                                             const uint32_t* epoch_base, int pass, uint32_t* op_mask)
 {
     const uint32_t epoch = *epoch_base + (uint32_t)pass;
-    collect_tile<true, kBatchTileW, kBatchTileH, kBatchLdsSet>(g, ops[blockIdx.z], epoch, (int)(epoch & 1u), op_mask,
-                                                               blockIdx.z);
+    collect_tile<true, kTW, kTH, kBatchLdsSet>(g, ops[blockIdx.z], epoch, (int)(epoch & 1u), op_mask, blockIdx.z);
 }
 
 // ---------------------------------------------------------------------------
@@ -1832,6 +1843,36 @@ int persistent_grid(const tsdf_grid* g)
     return n < 64 ? 64 : n;
 }
 
+bool small_image(const tsdf_grid* g)
+{
+    return (size_t)((g->p.width + 7) / 8) * ((g->p.height + 7) / 8) <= (size_t)kSmallPatches * g->n_cu;
+}
+
+dim3 tile_grid(const tsdf_grid* g, int tw, int th, int ops)
+{
+    return dim3((g->p.width + tw - 1) / tw, (g->p.height + th - 1) / th, ops);
+}
+
+void launch_collect(const tsdf_grid* g, const OpDesc& op, uint32_t epoch, int par, hipStream_t s)
+{
+    if (small_image(g))
+        hipLaunchKernelGGL((k_collect<8, 8>), tile_grid(g, 8, 8, 1), dim3(kThreads), 0, s, view(g), op, epoch, par);
+    else
+        hipLaunchKernelGGL((k_collect<kTileW, kTileH>), tile_grid(g, kTileW, kTileH, 1), dim3(kThreads), 0, s, view(g),
+                           op, epoch, par);
+}
+
+void launch_collect_batch(const tsdf_grid* g, const OpDesc* ops, int n_ops, const uint32_t* epoch_base, int pass,
+                          hipStream_t s)
+{
+    if (small_image(g))
+        hipLaunchKernelGGL((k_collect_batch<16, 16>), tile_grid(g, 16, 16, n_ops), dim3(kThreads), 0, s, view(g), ops,
+                           epoch_base, pass, g->op_mask);
+    else
+        hipLaunchKernelGGL((k_collect_batch<kBatchTileW, kBatchTileH>), tile_grid(g, kBatchTileW, kBatchTileH, n_ops),
+                           dim3(kThreads), 0, s, view(g), ops, epoch_base, pass, g->op_mask);
+}
+
 template <typename T>
 void launch_integrate(const tsdf_grid* g, const OpDesc& op, int par, hipStream_t s, bool color)
 {
@@ -2434,10 +2475,9 @@ tsdf_status tsdf_integrate(tsdf_grid* g, const uint16_t* depth, int32_t pitch, c
     const uint32_t epoch = ++g->epoch;
     ++g->map_gen;
     const int par = (int)(epoch & 1u);
-    const dim3 cgrid((g->p.width + kTileW - 1) / kTileW, (g->p.height + kTileH - 1) / kTileH);
     {
         ProfScope ps(g, s, TSDF_K_COLLECT);
-        hipLaunchKernelGGL(k_collect, cgrid, dim3(kThreads), 0, s, view(g), op, epoch, par);
+        launch_collect(g, op, epoch, par, s);
     }
     const bool color = g->p.with_color != 0;
     {
@@ -2464,11 +2504,10 @@ void enqueue_batch_passes(tsdf_grid* g, int n_ops, int per, hipStream_t s, bool 
     const uint32_t* ep = &g->stage_dev->epoch_base;
     for (int cb = 0, pass = 0; cb < n_ops; cb += per, ++pass) {
         const int n = (n_ops - cb) < per ? (n_ops - cb) : per;
-        const dim3 cgrid((g->p.width + kBatchTileW - 1) / kBatchTileW, (g->p.height + kBatchTileH - 1) / kBatchTileH, n);
         const OpDesc* ops = g->stage_dev->ops + cb;
         {
             ProfScope ps(g, s, TSDF_K_COLLECT_BATCH, profile);
-            hipLaunchKernelGGL(k_collect_batch, cgrid, dim3(kThreads), 0, s, view(g), ops, ep, pass, g->op_mask);
+            launch_collect_batch(g, ops, n, ep, pass, s);
         }
         {
             ProfScope ps(g, s, TSDF_K_INTEGRATE_BATCH, profile);
