@@ -1734,6 +1734,7 @@ struct tsdf_grid {
     size_t sort_tmp_cap;  // bytes
     void* mc_buf;         // marching cubes: edge masks, bricks' shares and sums, grown on demand
     size_t mc_cap;        // bytes
+    void* clean_buf;      // cleanMemory: counts, move lists and a flag per brick (allocated on first call)
 };
 
 namespace {
@@ -2388,6 +2389,7 @@ void tsdf_destroy(tsdf_grid* g)
     }
     (void)hipFree(g->sort_tmp);
     (void)hipFree(g->mc_buf);
+    (void)hipFree(g->clean_buf);
     if (g->stage_host)
         (void)hipHostFree(g->stage_host);
     if (g->staging_done)
