@@ -65,21 +65,38 @@ struct Sample {
     float wt[8];  // trilinear weights
 };
 
-// phi (and its gradient) at p; false where the field is undefined.
-// The lookups of the corners' blocks (all but the ray's own) are issued
-// together, then the 8 voxel loads, so a sample costs at most two round trips.
-// On success the ray's block is the nearest voxel's.
-template <typename T, bool kFull>
-__device__ __forceinline__ bool field_sample(const GridView& g, const float* sdf_ovr, float px, float py,
-                                             float pz, BrickCache& bc, Sample& smp)
+// The cell of 8 voxel centres around a position: its lower corner's voxel and
+// the position in it, 0..1 per axis.
+struct Cell {
+    int k[3];
+    float fr[3];
+};
+
+// The cell of p; false outside any addressable block (and for NaN).
+__device__ __forceinline__ bool cell_at(const GridView& g, const float (&p)[3], Cell& q)
 {
     const float rvl = 1.0f / g.vl;
-    const float ux = px * rvl - 0.5f, uy = py * rvl - 0.5f, uz = pz * rvl - 0.5f;
-    const float fx0 = floorf(ux), fy0 = floorf(uy), fz0 = floorf(uz);
-    if (!(fabsf(fx0) < 1.6e7f && fabsf(fy0) < 1.6e7f && fabsf(fz0) < 1.6e7f))
-        return false;  // outside any addressable block (and NaN)
-    const int kx = (int)fx0, ky = (int)fy0, kz = (int)fz0;
-    const float fr[3] = {ux - fx0, uy - fy0, uz - fz0};
+    bool ok = true;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        const float u = p[a] * rvl - 0.5f, f = floorf(u);
+        ok = ok && fabsf(f) < 1.6e7f;
+        q.k[a] = (int)f;
+        q.fr[a] = u - f;
+    }
+    return ok;
+}
+
+// The 8 voxels of a cell; false where the field is undefined.
+// The lookups of the corners' blocks (all but the ray's own) are issued
+// together, then the 8 voxel loads, so a cell costs at most two round trips.
+// On success the ray's block is the voxel's nearest to the position.
+template <typename T>
+__device__ __forceinline__ bool load_cell(const GridView& g, const float* sdf_ovr, const Cell& q, BrickCache& bc,
+                                          uint32_t (&idx)[8], float (&V)[8])
+{
+    const int kx = q.k[0], ky = q.k[1], kz = q.k[2];
+    const float(&fr)[3] = q.fr;
     const int bx[2] = {kx >> 3, (kx + 1) >> 3}, by[2] = {ky >> 3, (ky + 1) >> 3}, bz[2] = {kz >> 3, (kz + 1) >> 3};
     const bool two[3] = {bx[1] != bx[0], by[1] != by[0], bz[1] != bz[0]};
     uint32_t key[8];
@@ -121,23 +138,38 @@ __device__ __forceinline__ bool field_sample(const GridView& g, const float* sdf
     if (!all)
         return false;
     const T* pay = (const T*)g.payload;
-    float V[8], w[8];
+    float w[8];
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
         const int ax = c & 1, ay = (c >> 1) & 1, az = (c >> 2) & 1;
         const int v = ((kx + ax) & 7) + 8 * ((ky + ay) & 7) + 64 * ((kz + az) & 7);
-        smp.idx[c] = (uint32_t)bid[c] * (uint32_t)kVPB + (uint32_t)v;
+        idx[c] = (uint32_t)bid[c] * (uint32_t)kVPB + (uint32_t)v;
         ld_pair(pay + (size_t)bid[c] * (2 * kVPB), v, V[c], w[c]);
     }
     if (sdf_ovr)
 #pragma unroll
         for (int c = 0; c < 8; ++c)
-            V[c] = sdf_ovr[smp.idx[c]];
+            V[c] = sdf_ovr[idx[c]];
 #pragma unroll
     for (int c = 0; c < 8; ++c)
         all = all && w[c] > 0.0f;
     if (!all)
         return false;
+    const int near = (fr[0] >= 0.5f ? 1 : 0) | (fr[1] >= 0.5f ? 2 : 0) | (fr[2] >= 0.5f ? 4 : 0);
+    bc.bx = (near & 1) ? bx[1] : bx[0];
+    bc.by = (near & 2) ? by[1] : by[0];
+    bc.bz = (near & 4) ? bz[1] : bz[0];
+#pragma unroll
+    for (int c = 0; c < 8; ++c)
+        bc.id = near == c ? bid[c] : bc.id;
+    return true;
+}
+
+// phi (and its gradient) in a cell with the values V.
+template <bool kFull>
+__device__ __forceinline__ void interpolate(const GridView& g, const float (&fr)[3], const float (&V)[8], Sample& smp)
+{
+    const float rvl = 1.0f / g.vl;
     float s = 0.f, g0 = 0.f, g1 = 0.f, g2 = 0.f;
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
@@ -160,13 +192,18 @@ __device__ __forceinline__ bool field_sample(const GridView& g, const float* sdf
         smp.grad[1] = g1 * rvl;
         smp.grad[2] = g2 * rvl;
     }
-    const int near = (fr[0] >= 0.5f ? 1 : 0) | (fr[1] >= 0.5f ? 2 : 0) | (fr[2] >= 0.5f ? 4 : 0);
-    bc.bx = (near & 1) ? bx[1] : bx[0];
-    bc.by = (near & 2) ? by[1] : by[0];
-    bc.bz = (near & 4) ? bz[1] : bz[0];
-#pragma unroll
-    for (int c = 0; c < 8; ++c)
-        bc.id = near == c ? bid[c] : bc.id;
+}
+
+// phi (and its gradient) at p; false where the field is undefined.
+template <typename T, bool kFull>
+__device__ __forceinline__ bool field_sample(const GridView& g, const float* sdf_ovr, const float (&p)[3],
+                                             BrickCache& bc, Sample& smp)
+{
+    Cell q;
+    float V[8];
+    if (!cell_at(g, p, q) || !load_cell<T>(g, sdf_ovr, q, bc, smp.idx, V))
+        return false;
+    interpolate<kFull>(g, q.fr, V, smp);
     return true;
 }
 
@@ -187,10 +224,12 @@ __device__ __forceinline__ Ray make_ray(const ViewPose& P, const RenderCam& cam,
     return r;
 }
 
-// What one ray of a march keeps: the exact quotients by its direction
-// (quot_rn), the two fixed steps.
+// What one ray of a march keeps: the exact quotients by its direction and its
+// length (quot_rn), the two fixed steps.  An axis the ray does not move along
+// has the quotient 0 and the exit +inf, so exit_step needs no branch.
 struct RayGeom {
-    double Rd[3];
+    double Rd[3], Rn;
+    float never[3];    // +inf on an axis without an exit, else 0
     float ustep, eps;  // the step where the field is undefined, and past a block's face
 };
 
@@ -209,7 +248,7 @@ __device__ __forceinline__ float exit_step(const GridView& g, const Ray& r, cons
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
         const float e = (float)(b[a] + (r.d[a] > 0.f ? 1 : 0)) * g.vbl - r.o[a];
-        te = r.d[a] != 0.f ? fminf(te, quot_rn(e, q.Rd[a])) : te;
+        te = fminf(te, quot_rn(e, q.Rd[a]) + q.never[a]);
     }
     return fmaxf(te - lam + q.eps, q.eps);
 }
@@ -228,18 +267,21 @@ __device__ __forceinline__ float ld_weight(const __half* b, int v) { return __ha
 //    one hits (the voxel nearest to a position lies in the position's block,
 //    up to the rounding that the half voxel between them absorbs for
 //    coordinates below 2^20 voxels, so the field is undefined there);
-//  - inside a block, the weight of the voxel nearest to each of the next
-//    kRWalk positions is loaded; where it is not positive the field is
-//    undefined (that voxel is one of the position's 8) and the step is
-//    taken, else the whole sample is.
+//  - inside a block, the weight of the voxel each of the next kRWalk
+//    positions is in is loaded; where it is not positive the field is
+//    undefined (that voxel, floor(p / vl), is one of the position's 8: its
+//    lower corner floor(p / vl - 0.5) or the next along each axis, rounded or
+//    not) and the step is taken, else the whole sample is.
 // Before lam_near and from lam_far on no brick holds a position of the ray
 // (the tile bounds), so the first stretch makes no lookups and the march ends
 // at lam_far.  Every position and sample is that of the plain march.
 //
-// Bound by the round trips of the longest rays (about 165 rounds of up to 4 of
-// them; the mean ray takes 18), not by bytes.  16 views of 320 x 240 (1.2 M
-// rays): 4.69 -> 1.23 ms; one of 640 x 480: 1.84 -> 0.61 ms.  Looking 2 blocks
-// and 4 samples ahead is the best of 1 .. 8 each (8 and 8: 1.67 and 0.90 ms).
+// Bound by the longest wavefronts, not by bytes: 190 rounds of about 3 us, each
+// up to 4 round trips and 700 instructions, where the mean one takes 25.
+// 16 views of 320 x 240 (1.2 M rays): 4.69 -> 1.12 ms; one of 640 x 480:
+// 1.84 -> 0.55 ms.  Looking 2 blocks and 4 samples ahead is the best over all
+// sizes (1 and 3: 0.53 and 1.11 ms, but 160 x 120 0.58 -> 0.63; 8 and 8: 0.90
+// and 1.67).
 #ifndef TSDF_RENDER_LOOK
 #define TSDF_RENDER_LOOK 2
 #endif
@@ -263,8 +305,11 @@ __device__ __forceinline__ RayGeom ray_geom(const GridView& g, const Ray& r)
 {
     RayGeom q;
 #pragma unroll
-    for (int a = 0; a < 3; ++a)
-        q.Rd[a] = 1.0 / (double)r.d[a];
+    for (int a = 0; a < 3; ++a) {
+        q.Rd[a] = r.d[a] != 0.f ? 1.0 / (double)r.d[a] : 0.0;
+        q.never[a] = r.d[a] != 0.f ? 0.f : INFINITY;
+    }
+    q.Rn = 1.0 / (double)r.dn;
     q.ustep = kRMinStepVox * g.vl / r.dn;
     q.eps = 1e-3f * g.vl / r.dn;
     return q;
@@ -349,22 +394,19 @@ __device__ float trace(const GridView& g, const float* sdf_ovr, const RenderCam&
             if (known && lam < lim && step < kRenderMaxSteps) {
                 // in block bc: the nearest voxel's weight, kRWalk positions ahead
                 const T* brick = (const T*)g.payload + (size_t)bc.id * (2 * kVPB);
+                const float fb0 = (float)bc.bx, fb1 = (float)bc.by, fb2 = (float)bc.bz;
                 float lu[kRWalk + 1], w[kRWalk];
                 bool in[kRWalk], own[kRWalk];
                 lu[0] = lam;
 #pragma unroll
                 for (int k = 0; k < kRWalk; ++k) {
                     const float p[3] = {r.o[0] + lu[k] * r.d[0], r.o[1] + lu[k] * r.d[1], r.o[2] + lu[k] * r.d[2]};
-                    int v[3];
-#pragma unroll
-                    for (int a = 0; a < 3; ++a) {
-                        const float u = p[a] * rvl - 0.5f, f = floorf(u);
-                        v[a] = (int)f + (u - f >= 0.5f ? 1 : 0);
-                    }
-                    in[k] = (int)floorf(p[0] * g.rvbl) == bc.bx && (int)floorf(p[1] * g.rvbl) == bc.by &&
-                            (int)floorf(p[2] * g.rvbl) == bc.bz;
-                    own[k] = (v[0] >> 3) == bc.bx && (v[1] >> 3) == bc.by && (v[2] >> 3) == bc.bz;
-                    w[k] = ld_weight(brick, (v[0] & 7) + 8 * (v[1] & 7) + 64 * (v[2] & 7));
+                    const int x = (int)floorf(p[0] * rvl) - 8 * bc.bx, y = (int)floorf(p[1] * rvl) - 8 * bc.by,
+                              z = (int)floorf(p[2] * rvl) - 8 * bc.bz;
+                    in[k] = floorf(p[0] * g.rvbl) == fb0 && floorf(p[1] * g.rvbl) == fb1 &&
+                            floorf(p[2] * g.rvbl) == fb2;
+                    own[k] = (unsigned)(x | y | z) < 8u;
+                    w[k] = ld_weight(brick, (x + 8 * y + 64 * z) & (kVPB - 1));
                     lu[k + 1] = lu[k] + q.ustep;
                 }
                 bool go = true;
@@ -380,8 +422,8 @@ __device__ float trace(const GridView& g, const float* sdf_ovr, const RenderCam&
         }
         __builtin_amdgcn_wave_barrier();
         if (due) {
-            const bool valid = field_sample<T, false>(g, sdf_ovr, r.o[0] + lam * r.d[0], r.o[1] + lam * r.d[1],
-                                                      r.o[2] + lam * r.d[2], bc, smp);
+            const float p[3] = {r.o[0] + lam * r.d[0], r.o[1] + lam * r.d[1], r.o[2] + lam * r.d[2]};
+            const bool valid = field_sample<T, false>(g, sdf_ovr, p, bc, smp);
             const float phi = smp.phi;
             hit = valid && prev_valid && prev_phi > 0.f && phi <= 0.f;
             if (hit) {
@@ -389,8 +431,7 @@ __device__ float trace(const GridView& g, const float* sdf_ovr, const RenderCam&
             } else {
                 float st;
                 if (valid) {
-                    const float m = kRStepFrac * fabsf(phi);
-                    st = fmaxf(m, kRMinStepVox * vl) / r.dn;
+                    st = quot_rn(fmaxf(kRStepFrac * fabsf(phi), kRMinStepVox * vl), q.Rn);
                 } else {
                     int b[3];
                     ray_block(g, r, lam, b);
@@ -423,28 +464,39 @@ __device__ float trace(const GridView& g, const float* sdf_ovr, const RenderCam&
     float a = prev_lam, b = lam;
     const float fa = prev_phi;
     float x = (fb == 0.f) ? b : b - fb * (b - a) / (fb - fa);
-    for (int it = 0; it < kRootIters; ++it) {
-        if (!field_sample<T, true>(g, sdf_ovr, r.o[0] + x * r.d[0], r.o[1] + x * r.d[1],
-                                   r.o[2] + x * r.d[2], bc, smp))
-            return 0.f;
+    // The iterations stay within a step of the march and mostly in one cell,
+    // whose 8 values are kept: a wavefront takes 12 of them (its slowest ray).
+    // 16 views of 320 x 240 1.23 -> 1.18 ms.
+    Cell at = {{0, 0, 0}, {0.f, 0.f, 0.f}};
+    float V[8];
+    bool loaded = false, ok = true, done = false, last = false;
+    for (int it = 1; ok && !last; ++it) {
+        Cell q;
+        const float p[3] = {r.o[0] + x * r.d[0], r.o[1] + x * r.d[1], r.o[2] + x * r.d[2]};
+        ok = cell_at(g, p, q);
+        if (ok && !(loaded && q.k[0] == at.k[0] && q.k[1] == at.k[1] && q.k[2] == at.k[2])) {
+            ok = load_cell<T>(g, sdf_ovr, q, bc, smp.idx, V);
+            loaded = true;
+        }
+        at = q;
+        interpolate<true>(g, q.fr, V, smp);
         const float fx = smp.phi;
-        if (fx == 0.f)
-            break;
-        if (fx > 0.f)
-            a = x;
-        else
-            b = x;
-        const float s = smp.grad[0] * r.d[0] + smp.grad[1] * r.d[1] + smp.grad[2] * r.d[2];
-        float nx = (s < 0.f) ? x - fx / s : 0.5f * (a + b);
-        if (!(nx > a && nx < b))
-            nx = 0.5f * (a + b);
-        const float dx = fabsf(nx - x);
-        x = nx;
-        if (dx <= 2e-7f * (1.0f + x))
-            break;
+        last = done || fx == 0.f;
+        if (ok && !last) {
+            if (fx > 0.f)
+                a = x;
+            else
+                b = x;
+            const float s = smp.grad[0] * r.d[0] + smp.grad[1] * r.d[1] + smp.grad[2] * r.d[2];
+            float nx = (s < 0.f) ? x - fx / s : 0.5f * (a + b);
+            if (!(nx > a && nx < b))
+                nx = 0.5f * (a + b);
+            const float dx = fabsf(nx - x);
+            x = nx;
+            done = dx <= 2e-7f * (1.0f + x) || it == kRootIters;  // the sample at x is the last
+        }
     }
-    if (!field_sample<T, true>(g, sdf_ovr, r.o[0] + x * r.d[0], r.o[1] + x * r.d[1], r.o[2] + x * r.d[2],
-                               bc, smp))
+    if (!ok)
         return 0.f;
     const float s = smp.grad[0] * r.d[0] + smp.grad[1] * r.d[1] + smp.grad[2] * r.d[2];
     const float gn = sqrtf(smp.grad[0] * smp.grad[0] + smp.grad[1] * smp.grad[1] + smp.grad[2] * smp.grad[2]);
@@ -563,7 +615,7 @@ __device__ __forceinline__ bool pixel_jacobian(const GridView& g, const float* s
 {
     BrickCache bc = {0, 0, 0, -1};
     const float p[3] = {r.o[0] + lam * r.d[0], r.o[1] + lam * r.d[1], r.o[2] + lam * r.d[2]};
-    if (!field_sample<T, true>(g, sdf_ovr, p[0], p[1], p[2], bc, smp))
+    if (!field_sample<T, true>(g, sdf_ovr, p, bc, smp))
         return false;
     s = smp.grad[0] * r.d[0] + smp.grad[1] * r.d[1] + smp.grad[2] * r.d[2];
     if (!(s < 0.f))
