@@ -125,7 +125,9 @@ typedef struct {
     int32_t raycast_budget;       /* march rounds of a ray before it is handed  */
                                   /* to a second kernel that carries each ray   */
                                   /* with 16 lanes (results do not depend on    */
-                                  /* it); 0 = never, at most 4096               */
+                                  /* it); 0 = never, at most 4096.  Large images */
+                                  /* over fine grids keep every ray: wavefronts */
+                                  /* x max_ray_length / block side >= 2.1e6     */
 } tsdf_tuning;
 
 /* Camera of a render view (the differentiable render has its own resolution
@@ -294,7 +296,8 @@ tsdf_status tsdf_export_bricks(tsdf_grid *g, int32_t *coords, float *sdf, float 
 /* GPUVoxelGrid::cleanMemory(space), GPUVoxelGrid.cpp:185-196 with cleanTag
  * :785-805: erases every brick whose 512 weights are all zero (the surviving
  * bricks are compacted and the table rebuilt).  Synchronous; *n_removed (or
- * NULL) receives the number erased. */
+ * NULL) receives the number erased.  Allocates 5 bytes per brick of the pool
+ * on the first call, kept with the grid. */
 tsdf_status tsdf_clean(tsdf_grid *g, uint64_t *n_removed, void *stream);
 
 /* Triangle mesh of the zero level set (stands in for marchingCubesHost,
