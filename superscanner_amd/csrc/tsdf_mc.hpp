@@ -346,7 +346,10 @@ __device__ __forceinline__ unsigned long long mc_key(int gx, int gy, int gz, int
 // Loads the voxels kLo .. 8 of brick b along each axis, from the brick and its
 // neighbours, into tile (s, w), x fastest; a voxel of a missing or
 // never-written brick reads (0, 0).  nb: the bricks at block offsets kLo / 8
-// .. 1 (-1 where missing), x fastest.  Starts and ends with a barrier.
+// .. 1 (-1 where missing), x fastest.  A lookup compares 32-bit keys, and a
+// missing block's key may be that of a brick elsewhere (alias_vector): the
+// brick found is the neighbour only if its block is the one asked for.
+// Starts and ends with a barrier.
 template <typename T, int kLo, int kN>
 __device__ void mc_load_tile(const GridView& g, unsigned int b, float2* tile, int* nb, int4& bc)
 {
@@ -357,8 +360,11 @@ __device__ void mc_load_tile(const GridView& g, unsigned int b, float2* tile, in
         const int dx = c % bs + first, dy = c / bs % bs + first, dz = c / (bs * bs) + first;
         const int4 at = g.coords[b];
         int id = (dx | dy | dz) == 0 ? (int)b : find_brick(g, at.x + dx, at.y + dy, at.z + dz);
-        if (id >= 0 && (g.coords[id].w & 1))
-            id = -1;
+        if (id >= 0) {
+            const int4 q = g.coords[id];
+            if ((q.w & 1) || q.x != at.x + dx || q.y != at.y + dy || q.z != at.z + dz)
+                id = -1;
+        }
         nb[c] = id;
         if (c == 0)
             bc = at;
