@@ -560,10 +560,14 @@ __device__ __forceinline__ void view_stretch(const GridView& g, const RenderArgs
     }
     if (!alias_free(bmin, bmax, plo, phi))
         return;
-    const float zt = tb_depth(a.tb.z[((size_t)view * a.tb.tiles_y + i / kTbTile) * a.tb.tiles_x + j / kTbTile],
-                              a.tb.epoch);
-    const float zf = tb_far(a.tb.zf[((size_t)view * a.tb.far_y + i / kTbFarTile) * a.tb.far_x + j / kTbFarTile],
-                            a.tb.epoch);
+    const unsigned long long ez = a.tb.z[((size_t)view * a.tb.tiles_y + i / kTbTile) * a.tb.tiles_x + j / kTbTile];
+    const unsigned long long ef = a.tb.zf[((size_t)view * a.tb.far_y + i / kTbFarTile) * a.tb.far_x + j / kTbFarTile];
+    // A newer stamp: a call on another stream has overwritten the entry, which
+    // may have been this call's (an entry with this call's stamp is whole: the
+    // newer one wins both the minimum and the maximum).  No bound then.
+    if ((int)(~(uint32_t)(ez >> 32) - a.tb.epoch) > 0 || (int)((uint32_t)(ef >> 32) - a.tb.epoch) > 0)
+        return;
+    const float zt = tb_depth(ez, a.tb.epoch), zf = tb_far(ef, a.tb.epoch);
     lam_near = zt * (1.0f - 1e-4f) - 1e-4f;
     lam_far = zf * (1.0f + 1e-4f) + 1e-4f;
 }
@@ -912,7 +916,8 @@ tsdf_status ensure_reduce(tsdf_grid* g, size_t part, size_t rec, size_t tmp)
 // over them.  Left out (a.tb.z null: the march looks everything up) where the
 // bound on a position's error leaves no depth to clip at, where a pose is too
 // far from rigid for its inverse to be its transpose, and while the stream is
-// captured (a replay would reuse the bounds' call stamp).
+// captured (a replay would reuse the bounds' call stamp).  Calls that overlap
+// on one grid share the maps: see view_stretch.
 tsdf_status view_bounds(tsdf_grid* g, int32_t n_views, const float* E, RenderArgs& a, hipStream_t s)
 {
     double tmax = 0.0, skew = 0.0;
