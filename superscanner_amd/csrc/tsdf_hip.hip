@@ -71,29 +71,50 @@ struct Offsets {
 constexpr int kThreads = 256;
 // Collection tiles (pixels of a workgroup, in 8 x 8 patches) and their block
 // sets.  A set holds kLdsSet blocks; a full one falls back to claiming blocks
-// one by one, which costs far more than the set.  Large images take 32 x 8
-// pixels, a patch per wavefront; images of at most kSmallPatches patches a CU
-// take one patch a workgroup: fewer workgroups than that leave the chip idle,
-// and the patches of a small image are wide, with hundreds of blocks each.
-// Collection, 64 x 8 / 32 x 8 / 16 x 16 / 8 x 8 pixels a tile:
-//   160 x 120 (300 patches, 5 mm voxels)      75    31    25    14 us
-//   320 x 180 (920, 2 mm)                    112    62    62    28
-//   320 x 240 (1 200, 5 mm)                   34    17    16    18
-//   848 x 480 (6 360, 4 mm)                   27    25    25    44
-//   1280 x 720 (14 400, 2 mm)                 95    54    56   130
+// one by one, which costs far more than the set.  A wide tile sees a block
+// fewer times (fewer claims, above all where a map grows); a narrow one makes
+// more workgroups and keeps its set from filling up.  So:
+//  - images of at most kSmallPatches patches a CU take one patch a workgroup:
+//    fewer workgroups than that leave the chip idle, and their patches are
+//    wide, with hundreds of blocks each;
+//  - 32 x 8 pixels, a patch per wavefront, up to kNarrowPatches patches a CU,
+//    and where a block is less than kFineBlock pixels wide at 1 m (many blocks
+//    a tile);
+//  - else 64 x 8.
+// Collection in us, 64 x 8 / 32 x 8 / 8 x 8 pixels a tile (the same for the
+// frames that fill an empty map):
+//   160 x 120 (300 patches, 5 mm voxels)    78   34   14    (119   57   35)
+//   320 x 180 (920, 2 mm)                  111   61   28    (323  228  139)
+//   320 x 240 (1 200, 4 mm)                 28   18   21     (36   29   40)
+//   480 x 360 (2 700, 5 mm)                 19   16          (43   37)
+//   548 x 412 (3 588, 5 mm)                 19   17.5        (41   40)
+//   576 x 432 (3 888, 5 mm; 15 px a block)  18.5 17.7        (39   42)
+//   848 x 480 (6 360, 4 mm; 14)             25   24          (37   41)
+//   1280 x 720 (14 400, 4 mm; 21)           32   35          (50   64)
+//   641 x 479 (4 860, 4 mm; 10)             25   21          (35   36)
+//   848 x 480 (6 360, 2 mm; 7)              78   45         (223  167)
+//   1280 x 720 (14 400, 2 mm; 10)           57   54         (201  231)
+// A live scan (1 to 2 % of the blocks new): 848 x 480 at 4 mm 31.8 / 30.8 over
+// 120 frames, 25.9 / 26.6 over 600; 1280 x 720 at 2 mm 181 / 151.
 #ifndef TSDF_TILE_W
-#define TSDF_TILE_W 32
+#define TSDF_TILE_W 64
 #endif
 #ifndef TSDF_TILE_H
 #define TSDF_TILE_H 8
+#endif
+#ifndef TSDF_TILE_W_NARROW
+#define TSDF_TILE_W_NARROW 32
 #endif
 #ifndef TSDF_LDS_SET
 #define TSDF_LDS_SET 1024
 #endif
 constexpr int kTileW = TSDF_TILE_W;
 constexpr int kTileH = TSDF_TILE_H;
+constexpr int kTileWNarrow = TSDF_TILE_W_NARROW;
 constexpr int kLdsSet = TSDF_LDS_SET;
 constexpr int kSmallPatches = 4;
+constexpr int kNarrowPatches = 14;
+constexpr float kFineBlock = 12.0f;
 // A batch pass collects several ops at once (grid.z = op), which fills the
 // GPU with larger tiles; larger tiles also see a block fewer times per op.
 // 8 ops, 64 x 16 / 16 x 16 pixels: 848 x 480 89 / 104 us, 424 x 240 47 / 44,
@@ -1851,9 +1872,19 @@ int persistent_grid(const tsdf_grid* g)
     return n < 64 ? 64 : n;
 }
 
+size_t image_patches(const tsdf_grid* g)
+{
+    return (size_t)((g->p.width + 7) / 8) * ((g->p.height + 7) / 8);
+}
+
 bool small_image(const tsdf_grid* g)
 {
-    return (size_t)((g->p.width + 7) / 8) * ((g->p.height + 7) / 8) <= (size_t)kSmallPatches * g->n_cu;
+    return image_patches(g) <= (size_t)kSmallPatches * g->n_cu;
+}
+
+bool narrow_tiles(const tsdf_grid* g)
+{
+    return image_patches(g) <= (size_t)kNarrowPatches * g->n_cu || g->cam.fx * g->vbl < kFineBlock;
 }
 
 dim3 tile_grid(const tsdf_grid* g, int tw, int th, int ops)
@@ -1865,6 +1896,9 @@ void launch_collect(const tsdf_grid* g, const OpDesc& op, uint32_t epoch, int pa
 {
     if (small_image(g))
         hipLaunchKernelGGL((k_collect<8, 8>), tile_grid(g, 8, 8, 1), dim3(kThreads), 0, s, view(g), op, epoch, par);
+    else if (narrow_tiles(g))
+        hipLaunchKernelGGL((k_collect<kTileWNarrow, kTileH>), tile_grid(g, kTileWNarrow, kTileH, 1), dim3(kThreads), 0, s,
+                           view(g), op, epoch, par);
     else
         hipLaunchKernelGGL((k_collect<kTileW, kTileH>), tile_grid(g, kTileW, kTileH, 1), dim3(kThreads), 0, s, view(g),
                            op, epoch, par);
