@@ -14,7 +14,8 @@ The tunables are the fields of ``tsdf_tuning`` (include/tsdf.h):
   raycast_skip          exact empty-space skip of the raycast (0 none, 1 distance
                         field over superblocks, 2 depth bounds of image tiles)
   raycast_budget        march rounds of a ray before a second kernel carries it
-                        with 16 lanes (0 never)
+                        with 16 lanes (0 never; the default 12 only where
+                        the grid's size lets it pay, other values always)
   raycast_order         dispatch order of the raycast's tiles (slowest of the
                         previous raycast first, reversed, or the hardware's)
 

@@ -2090,23 +2090,9 @@ void launch_raycast(tsdf_grid* g, const Pose& P, float* points, float* colors, f
     rp.use_sb = g->tune.raycast_skip == 1;
     rp.use_tb = g->tune.raycast_skip == 2 && !kStats;
     // the group march replays no superblock distance field
-    rp.budget = (kStats || rp.use_sb) ? 0 : g->tune.raycast_budget;
-    // Whether rays are deferred.  One round of the 16-lane march looks up 16
-    // positions of a ray with 16 lanes' work, the per-lane march 4 with one:
-    // deferring pays while the chip has lanes to spare, and costs once it has
-    // none.  What a raycast has to do is bounded by the lookups of an empty
-    // march, wavefronts x d_max / vbl.  Raycast without and with deferral:
-    //   75 k   (160 x 120, 40 mm bricks)    269   135 us
-    //   575 k  (320 x 180, 16 mm)           571   375
-    //   1.2 M  (640 x 480, 40 mm)           275   209
-    //   2.0 M  (848 x 480, 32 mm)           180   143
-    //   2.25 M (640 x 360, 16 mm)           733  1006
-    //   3.6 M  (1280 x 720, 40 mm)          302   464
-    //   4.5 M  (1280 x 720, 32 mm)          234   272
-    //   9.0 M  (1280 x 720, 16 mm)         1319  3390
-    const double lookups = (double)((rp.W + 7) / 8) * ((rp.H + 7) / 8) * (rp.dmax / rp.vbl);
-    if (!(lookups < 2.1e6))
-        rp.budget = 0;
+    rp.budget = (kStats || rp.use_sb)
+                    ? 0
+                    : raycast_budget(g->tune.raycast_budget, rp.W, rp.H, rp.dmax, rp.vbl, g->n_cu);
     rp.lc = nullptr;  // the kernel points it at its LDS cache (TSDF_RAY_CACHE)
     const int qpar = (int)(g->ray_qepoch & 1u);
     if (rp.budget > 0)
@@ -2782,7 +2768,7 @@ void tsdf_default_tuning(tsdf_tuning* t)
         return;
     t->raycast_xcd_map = 0;
     t->raycast_skip = 2;
-    t->raycast_budget = 12;
+    t->raycast_budget = kDefaultBudget;
     t->integrate_wg_per_cu = 6;
     t->batch_ops_per_pass = 8;
     t->batch_graph = 1;

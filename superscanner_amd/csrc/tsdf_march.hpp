@@ -599,6 +599,33 @@ struct RayState {
 };
 static_assert(sizeof(RayState) == 64, "one 64-byte record per deferred ray");
 
+// The budget of a raycast: rounds of the per-lane march before a ray is
+// deferred, 0 for never.  A budget the caller has set is taken as it is; the
+// default one defers only while the chip has lanes to spare.  One round of the
+// 16-lane march looks up 16 positions of a ray with 16 lanes' work, the
+// per-lane march kSkipLook with one.  What a raycast has to do is bounded by
+// the lookups of an empty march, wavefronts x d_max / vbl: a coarse measure
+// (what the rays meet counts too), with the line past the largest image that
+// gains.  Raycast in us without and with deferral, 256 CUs:
+//   lookups a CU                                   never  deferred
+//     293   160 x 120, 40 mm bricks, open plane      269   135
+//   4 688   640 x 480, 40 mm, open plane             253   207
+//   6 216   533 x 300, 16 mm, rooms                  628   765
+//   7 764   848 x 480, 32 mm, room                   160   144
+//   7 969   960 x 540, 40 mm, open plane             259   301
+//   8 276   900 x 600, 40 mm, open plane             266   321
+//   8 828   900 x 510, 32 mm, room                   167   167
+//   8 789   640 x 360, 16 mm, rooms                  700  1051
+//  12 268   1066 x 600, 32 mm, room                  189   221
+//  17 578   1280 x 720, 32 mm, room                  227   286
+constexpr int kDefaultBudget = 12;
+constexpr double kDeferLookups = 8200.0;  // a CU
+inline int raycast_budget(int budget, int W, int H, float dmax, float vbl, int n_cu)
+{
+    const double lookups = (double)((W + 7) / 8) * ((H + 7) / 8) * (dmax / vbl);
+    return budget != kDefaultBudget || lookups < kDeferLookups * n_cu ? budget : 0;
+}
+
 constexpr int kRayUbVoxelIndex = 1;  // TSDF_RAY_UB_VOXEL_INDEX
 constexpr int kRayUbMissingOut = 2;  // TSDF_RAY_UB_MISSING_OUT
 #ifndef TSDF_SKIP_LOOK
