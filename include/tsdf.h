@@ -222,7 +222,10 @@ tsdf_status tsdf_raycast(tsdf_grid *g, const float E_cam2world[16], float *point
  * 0 where no surface is found.  sdf: optional DEVICE [n_bricks][512] float
  * values that replace the stored sdf (brick order of tsdf_export_bricks),
  * NULL = the stored values (an override needs a grid of at most 2^23 - 1
- * bricks); weights always come from the map. */
+ * bricks); weights always come from the map.  tsdf_render and
+ * tsdf_track_normal_eq grow grid-owned scratch on need (16 bytes per 8 x 8
+ * pixels of all views), kept until the grid is destroyed; without room for it
+ * they run without, more slowly. */
 
 /* normals: DEVICE [n][h][w][3] unit gradient of the field, or NULL. */
 tsdf_status tsdf_render(tsdf_grid *g, int32_t n_views, const float *E, const tsdf_view *cam,
@@ -336,7 +339,8 @@ tsdf_status tsdf_extract_mesh(tsdf_grid *g, float *triangles, float *colors, uin
  * +-32767 blocks per axis are refused).  *n_vertices and *n_triangles (host)
  * receive the mesh's sizes; nothing is written unless both fit their
  * capacities.  Vertex order is not fixed from call to call; the vertex set
- * and the triangle multiset are.  Synchronous. */
+ * and the triangle multiset are.  Synchronous.  Grows grid-owned scratch on
+ * need (208 bytes per brick of the map), kept until the grid is destroyed. */
 tsdf_status tsdf_marching_cubes(tsdf_grid *g, double *vertices, double *vertex_colors, double *vertex_normals,
                                 int32_t *triangles, uint64_t *vertex_keys, uint64_t vertex_cap,
                                 uint64_t triangle_cap, uint64_t *n_vertices, uint64_t *n_triangles, void *stream);

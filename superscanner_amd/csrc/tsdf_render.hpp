@@ -915,8 +915,9 @@ tsdf_status ensure_reduce(tsdf_grid* g, size_t part, size_t rec, size_t tmp)
 // The tile depth bounds of the views of `a`, made on stream s before a march
 // over them.  Left out (a.tb.z null: the march looks everything up) where the
 // bound on a position's error leaves no depth to clip at, where a pose is too
-// far from rigid for its inverse to be its transpose, and while the stream is
-// captured (a replay would reuse the bounds' call stamp).  Calls that overlap
+// far from rigid for its inverse to be its transpose, where the card has no
+// room for the maps (16 bytes per 64 pixels), and while the stream is captured
+// (a replay would reuse the bounds' call stamp).  Calls that overlap
 // on one grid share the maps: see view_stretch.
 tsdf_status view_bounds(tsdf_grid* g, int32_t n_views, const float* E, RenderArgs& a, hipStream_t s)
 {
@@ -960,8 +961,16 @@ tsdf_status view_bounds(tsdf_grid* g, int32_t n_views, const float* E, RenderArg
             g->vb[k] = nullptr;
         }
         g->vb_cap = 0;
-        for (int k = 0; k < 2; ++k)
-            HIPC(hipMalloc(&g->vb[k], nt * n_views * sizeof(unsigned long long)));
+        for (int k = 0; k < 2; ++k) {
+            const hipError_t e = hipMalloc(&g->vb[k], nt * n_views * sizeof(unsigned long long));
+            if (e == hipErrorOutOfMemory) {  // the maps only save time
+                (void)hipGetLastError();
+                (void)hipFree(g->vb[0]);
+                g->vb[0] = g->vb[1] = nullptr;
+                return TSDF_OK;
+            }
+            HIPC(e);
+        }
         // no entry carries a stamp yet (stamps start at 1)
         HIPC(hipMemset(g->vb[0], 0xFF, nt * n_views * sizeof(unsigned long long)));
         HIPC(hipMemset(g->vb[1], 0, nt * n_views * sizeof(unsigned long long)));
