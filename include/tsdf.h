@@ -125,11 +125,10 @@ typedef struct {
     int32_t raycast_budget;       /* march rounds of a ray before it is handed  */
                                   /* to a second kernel that carries each ray   */
                                   /* with 16 lanes (results do not depend on    */
-                                  /* it); 0 = never, at most 4096.  The default */
-                                  /* 12 defers on images and grids small enough */
-                                  /* for it to pay (wavefronts x max_ray_length */
-                                  /* / block side < 8200 a CU), any other value */
-                                  /* on all                                     */
+                                  /* it); 0 = never, at most 4096.  Images of 26 */
+                                  /* or more wavefronts (8 x 8 pixels) a CU, and */
+                                  /* of 6.5 or more where a raycast has no depth */
+                                  /* bounds, keep every ray: there it never pays */
 } tsdf_tuning;
 
 /* Camera of a render view (the differentiable render has its own resolution

@@ -14,8 +14,7 @@ The tunables are the fields of ``tsdf_tuning`` (include/tsdf.h):
   raycast_skip          exact empty-space skip of the raycast (0 none, 1 distance
                         field over superblocks, 2 depth bounds of image tiles)
   raycast_budget        march rounds of a ray before a second kernel carries it
-                        with 16 lanes (0 never; the default 12 only where
-                        the grid's size lets it pay, other values always)
+                        with 16 lanes (0 never; large images never do)
   raycast_order         dispatch order of the raycast's tiles (slowest of the
                         previous raycast first, reversed, or the hardware's)
 
@@ -98,13 +97,26 @@ def tune_integrate(grid, depths, poses, *, wg_per_cu=INTEGRATE_WG_PER_CU, rounds
     return {"integrate_wg_per_cu": wg}, table
 
 
+def defers(skip, W, H, n_cu):
+    """Whether a raycast of W x H pixels defers rays at all (raycast_budget in
+    tsdf_march.hpp): below 26 wavefronts a CU with the depth bounds of image
+    tiles (skip 2), below 6.5 without."""
+    waves = ((W + 7) // 8) * ((H + 7) // 8)
+    return skip != 1 and 2 * waves < (52 if skip == 2 else 13) * n_cu
+
+
 def tune_raycast(grid, poses, *, xcd_map=(0,), skip=(0, 1, 2), order=(0, 2), budget=(0, 12, 16), rounds=3):
     """Picks raycast_xcd_map, raycast_skip, raycast_order and raycast_budget
     for ``grid.raycast`` (the group march replays no superblock field, so
-    skip 1 runs without a budget).  The candidates are timed in `rounds`
+    skip 1 runs without a budget, and so do images too large for deferral,
+    defers()).  The candidates are timed in `rounds`
     interleaved rounds and each keeps its best time.  Returns (best tuning
     dict, [(xcd_map, skip, order, budget, ms), ...])."""
-    cands = [c for c in itertools.product(xcd_map, skip, order, budget) if not (c[1] == 1 and c[3])]
+    n_cu = torch.cuda.get_device_properties(grid.device).multi_processor_count
+    cands = [c for c in itertools.product(xcd_map, skip, order, budget)
+             if not c[3] or defers(c[1], grid.resj, grid.resi, n_cu)]
+    if not cands:  # only budgets that this image ignores were asked for
+        cands = list(itertools.product(xcd_map, skip, order, (0,)))
     best = {c: float("inf") for c in cands}
 
     def run():

@@ -1400,6 +1400,8 @@ void k_raycast(GridView g, Pose pose, RayParams rp, float* points, float* colors
             rq.use_sb = 0;
         }
     }
+    if (!rq.use_tb)
+        rq.budget = rq.budget_plain;
     unsigned int hit = 0, bad = 0, samples = 0, probes = 0;
     // the depth bound of this wavefront's 8 x 8 pixels (one tile of the map)
     float zt = -1.0f, zf = -1.0f;
@@ -2089,14 +2091,7 @@ void launch_raycast(tsdf_grid* g, const Pose& P, float* points, float* colors, f
         rp.order = 0;  // no previous raycast to order by yet
     rp.use_sb = g->tune.raycast_skip == 1;
     rp.use_tb = g->tune.raycast_skip == 2 && !kStats;
-    // the group march replays no superblock distance field
-    rp.budget = (kStats || rp.use_sb)
-                    ? 0
-                    : raycast_budget(g->tune.raycast_budget, rp.W, rp.H, rp.dmax, rp.vbl, g->n_cu);
     rp.lc = nullptr;  // the kernel points it at its LDS cache (TSDF_RAY_CACHE)
-    const int qpar = (int)(g->ray_qepoch & 1u);
-    if (rp.budget > 0)
-        ++g->ray_qepoch;
     rp.df = nullptr;
     for (int a = 0; a < 3; ++a)
         rp.df_lo[a] = rp.df_dim[a] = 0;
@@ -2109,6 +2104,13 @@ void launch_raycast(tsdf_grid* g, const Pose& P, float* points, float* colors, f
     TileBounds tb = tile_bounds(g, P);
     if (!(tb.z_lo > 1e-3f))
         rp.use_tb = 0;  // the drift bound leaves no depth to clip at
+    // the group march replays no superblock distance field
+    const int budget = (kStats || rp.use_sb) ? 0 : g->tune.raycast_budget;
+    rp.budget_plain = raycast_budget(budget, false, rp.W, rp.H, g->n_cu);
+    rp.budget = rp.use_tb ? raycast_budget(budget, true, rp.W, rp.H, g->n_cu) : rp.budget_plain;
+    const int qpar = (int)(g->ray_qepoch & 1u);
+    if (rp.budget > 0)
+        ++g->ray_qepoch;
     if (rp.use_tb) {
         tb.epoch = ++g->tb_epoch;
         const int nt = tb.tiles_x * tb.tiles_y;
@@ -2768,7 +2770,7 @@ void tsdf_default_tuning(tsdf_tuning* t)
         return;
     t->raycast_xcd_map = 0;
     t->raycast_skip = 2;
-    t->raycast_budget = kDefaultBudget;
+    t->raycast_budget = 12;
     t->integrate_wg_per_cu = 6;
     t->batch_ops_per_pass = 8;
     t->batch_graph = 1;

@@ -283,6 +283,7 @@ struct RayParams {
     int df_lo[3], df_dim[3];
     int use_tb;       // tile depth bounds replay allowed (alias certificate holds)
     int budget;       // rounds of the per-lane march before a ray is deferred (0: never)
+    int budget_plain;  // the same without tile bounds (use_tb 0 or no certificate)
     unsigned long long* lc;  // the workgroup's LDS cache of lookup results, or null
 };
 
@@ -600,30 +601,24 @@ struct RayState {
 static_assert(sizeof(RayState) == 64, "one 64-byte record per deferred ray");
 
 // The budget of a raycast: rounds of the per-lane march before a ray is
-// deferred, 0 for never.  A budget the caller has set is taken as it is; the
-// default one defers only while the chip has lanes to spare.  One round of the
-// 16-lane march looks up 16 positions of a ray with 16 lanes' work, the
-// per-lane march kSkipLook with one.  What a raycast has to do is bounded by
-// the lookups of an empty march, wavefronts x d_max / vbl: a coarse measure
-// (what the rays meet counts too), with the line past the largest image that
-// gains.  Raycast in us without and with deferral, 256 CUs:
-//   lookups a CU                                   never  deferred
-//     293   160 x 120, 40 mm bricks, open plane      269   135
-//   4 688   640 x 480, 40 mm, open plane             253   207
-//   6 216   533 x 300, 16 mm, rooms                  628   765
-//   7 764   848 x 480, 32 mm, room                   160   144
-//   7 969   960 x 540, 40 mm, open plane             259   301
-//   8 276   900 x 600, 40 mm, open plane             266   321
-//   8 828   900 x 510, 32 mm, room                   167   167
-//   8 789   640 x 360, 16 mm, rooms                  700  1051
-//  12 268   1066 x 600, 32 mm, room                  189   221
-//  17 578   1280 x 720, 32 mm, room                  227   286
-constexpr int kDefaultBudget = 12;
-constexpr double kDeferLookups = 8200.0;  // a CU
-inline int raycast_budget(int budget, int W, int H, float dmax, float vbl, int n_cu)
+// deferred, 0 for never.  One round of the 16-lane march looks up 16 positions
+// of a ray with 16 lanes' work, the per-lane march kSkipLook with one, so
+// deferring pays while the chip has lanes to spare: below 26 wavefronts of
+// pixels a CU with the tile bounds, and below 6.5 without them (then a ray
+// takes its budget in the empty space before the surface, and nearly all are
+// deferred).  Raycast in us without and with deferral, 256 CUs:
+//   with bounds      wavefronts a CU            without
+//   18.8  640 x 480 open plane  254  208         1.2  160 x 120 open plane  259  118
+//   23.9  720 x 540             253  242         4.7  320 x 240             249  188
+//   24.8  848 x 480 room        161  149         6.2  424 x 240 room        129  135
+//   28.3  900 x 510 room        167  167         6.3  426 x 240 16 mm       542  545
+//   31.9  960 x 540 open plane  259  301         7.4  400 x 300 open plane  247  251
+//   33.9  990 x 560 room        177  195        10.5  480 x 360             246  327
+//   56.3  1280 x 720 room       227  286        24.8  848 x 480 room        172  378
+inline int raycast_budget(int budget, bool bounds, int W, int H, int n_cu)
 {
-    const double lookups = (double)((W + 7) / 8) * ((H + 7) / 8) * (dmax / vbl);
-    return budget != kDefaultBudget || lookups < kDeferLookups * n_cu ? budget : 0;
+    const long long waves = (long long)((W + 7) / 8) * ((H + 7) / 8);
+    return 2 * waves < (bounds ? 52ll : 13ll) * n_cu ? budget : 0;
 }
 
 constexpr int kRayUbVoxelIndex = 1;  // TSDF_RAY_UB_VOXEL_INDEX

@@ -191,7 +191,7 @@ extern "C" int march_far_host(int H, int W, float fx, float fy, float cx, float 
     return 0;
 }
 
-extern "C" int budget_of(int budget, int W, int H, float dmax, float vbl, int n_cu)
+extern "C" int budget_of(int budget, int bounds, int W, int H, int n_cu)
 {
-    return raycast_budget(budget, W, H, dmax, vbl, n_cu);
+    return raycast_budget(budget, bounds != 0, W, H, n_cu);
 }

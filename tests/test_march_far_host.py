@@ -10,7 +10,7 @@ import numpy as np
 import pytest
 
 import oracle
-from superscanner_amd import synth
+from superscanner_amd import autotune, synth
 from test_march_host import HIPCC, ROOT, compare
 
 f, i, vp = C.c_float, C.c_int, C.c_void_p
@@ -26,7 +26,7 @@ def lib(tmp_path_factory):
                     os.path.join(ROOT, "tests", "cpp", "march_far_host.cpp")], check=True, capture_output=True)
     L = C.CDLL(str(so))
     L.march_far_host.argtypes = [i, i, f, f, f, f, f, f, f, i, vp, vp, vp, vp, C.c_uint32, vp, i, vp, vp, vp, vp]
-    L.budget_of.argtypes = [i, i, i, f, f, i]
+    L.budget_of.argtypes = [i, i, i, i, i]
     return L
 
 
@@ -80,11 +80,18 @@ def test_far_bound_and_deferred_state(lib, scene, budget):
 
 
 def test_rule_of_the_budget(lib):
-    """The default defers below 8 200 lookups of an empty march a CU; a budget
-    that the caller has set is taken at every size."""
-    sizes = [(160, 120, 0.04, True), (848, 480, 0.032, True), (640, 360, 0.016, False), (1280, 720, 0.016, False)]
-    for W, H, vbl, defers in sizes:
-        assert lib.budget_of(12, W, H, 10.0, vbl, 256) == (12 if defers else 0)
-        for b in (0, 1, 11, 16, 4096):
-            assert lib.budget_of(b, W, H, 10.0, vbl, 256) == b
-    assert lib.budget_of(12, 848, 480, 10.0, 0.032, 64) == 0  # a quarter of the CUs
+    """Rays are deferred below 26 wavefronts a CU with the tile bounds, below
+    6.5 without; the tuner times no budget that a raycast would ignore."""
+    for W, H, with_bounds, without in ((1, 1, 1, 1), (160, 120, 1, 1), (320, 328, 1, 1), (320, 337, 1, 0),
+                                       (848, 480, 1, 0), (832, 504, 1, 0), (832, 513, 0, 0), (1280, 720, 0, 0),
+                                       (16384, 16384, 0, 0)):
+        for b in (0, 1, 12, 4096):
+            assert lib.budget_of(b, 1, W, H, 256) == (b if with_bounds else 0), (W, H)
+            assert lib.budget_of(b, 0, W, H, 256) == (b if without else 0), (W, H)
+    assert lib.budget_of(12, 1, 848, 480, 64) == 0  # a quarter of the CUs
+    rng = np.random.default_rng(0)
+    for _ in range(200):
+        W, H, cu = int(rng.integers(1, 1500)), int(rng.integers(1, 1500)), int(rng.integers(1, 305))
+        for skip in (0, 2):
+            assert autotune.defers(skip, W, H, cu) == (lib.budget_of(12, skip == 2, W, H, cu) == 12)
+        assert not autotune.defers(1, W, H, cu)
