@@ -1468,7 +1468,10 @@ void k_raycast(GridView g, Pose pose, RayParams rp, float* points, float* colors
 // 848 x 480 and 47 us at 1280 x 720 over 650 k bricks; the far bound, at a
 // quarter of the tiles, costs 1 and 5 us of it and ends every ray that
 // leaves the map (160 x 120 over an open plane: raycast 447 -> 159 us).
-constexpr int kTbLdsTiles = 16384;  // 80 KiB of LDS: 1280 x 720 has 14 400 tiles, and two copies fit a CU
+// 80 KiB of LDS for both maps, so that two copies fit a CU (images of at most 8
+// rows or columns have half as many far tiles, up to 96 KiB, and one copy);
+// 1280 x 720 has 14 400 tiles.
+constexpr int kTbLdsTiles = 16384;
 #ifndef TSDF_TB_PER
 #define TSDF_TB_PER 128  // least bricks per workgroup run
 #endif

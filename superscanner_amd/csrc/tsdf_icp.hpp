@@ -501,6 +501,8 @@ __global__ __launch_bounds__(kIcpStepThreads) void k_icp_step(const double* part
         __hip_atomic_store(seen, kIcpEnded, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         return;
     }
+    if (report)  // now: the rest takes longer than the write
+        __hip_atomic_store(seen, report, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     const double nc = m[1];
     const double cx[3] = {m[2] / nc, m[3] / nc, m[4] / nc}, cy[3] = {m[5] / nc, m[6] / nc, m[7] / nc};
     const float rmse = sqrtf((float)(m[17] / nc));
@@ -536,8 +538,6 @@ __global__ __launch_bounds__(kIcpStepThreads) void k_icp_step(const double* part
         for (int k = 0; k < 16; ++k)
             st->best[k] = T[k];
     }
-    if (report)
-        __hip_atomic_store(seen, report, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // The sums into buf + kIcpBlocks * kIcpMoments (device), with buf's first

@@ -430,7 +430,7 @@ __device__ __forceinline__ V mc_block_scan(V v, V* lds, V* total)
     return v + before;
 }
 
-// Pass 1: every brick's triangles (two cells per thread), and the edges its
+// Pass 1: every brick's triangles (kVPB / kMcCountThreads cells per thread, four), and the edges its
 // cells use, set in the masks of the bricks that own them (cleared before).
 // `uses` counts the edge uses.  Bound by the chain coords -> lookups -> tile
 // of each brick: two wavefronts a brick keep more bricks in flight (room map,
