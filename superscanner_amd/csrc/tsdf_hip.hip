@@ -1464,8 +1464,9 @@ void k_raycast(GridView g, Pose pose, RayParams rp, float* points, float* colors
 // brick may cover in a copy of the tile maps in LDS, then merges its copy into
 // the global maps with one atomic per tile it touched.  Larger images than
 // kTbLdsTiles tiles go to the global maps directly.
-// Bound by a fixed chain (clear the copy, load, project, merge), 15 us at
-// 848 x 480 and 47 us at 1280 x 720 over 650 k bricks; the far bound, at a
+// Bound by a fixed chain (clear the copy, load, project, merge), 10 us at
+// 848 x 480 over 600 poses of the room, 15 (mean 18) between updates of scattered
+// frames, and 46 (mean 57) at 1280 x 720 over 650 k bricks; the far bound, at a
 // quarter of the tiles, costs 1 and 5 us of it and ends every ray that
 // leaves the map (160 x 120 over an open plane: raycast 447 -> 159 us).
 // 80 KiB of LDS for both maps, so that two copies fit a CU (images of at most 8

@@ -277,7 +277,8 @@ __device__ __forceinline__ float ld_weight(const __half* b, int v) { return __ha
 // at lam_far.  Every position and sample is that of the plain march.
 //
 // Bound by the longest wavefronts, not by bytes: 190 rounds of about 3 us, each
-// up to 4 round trips and 700 instructions, where the mean one takes 25.
+// up to 4 round trips and 700 instructions, where the mean one takes 25; with
+// many views also by issue, at 30 of 64 lanes (VALU 0.6 busy; one view 0.25).
 // 16 views of 320 x 240 (1.2 M rays): 4.69 -> 1.12 ms; one of 640 x 480:
 // 1.84 -> 0.55 ms.  Looking 2 blocks and 4 samples ahead is the best over all
 // sizes (1 and 3: 0.53 and 1.11 ms, but 160 x 120 0.58 -> 0.63; 8 and 8: 0.90
