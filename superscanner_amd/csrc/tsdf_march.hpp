@@ -862,9 +862,9 @@ __host__ __device__ __forceinline__ void lanes_meet()
 //    and k steps (each at most vbl per axis) move the reference's block index
 //    by at most k + 3 per axis, so steps 1 .. d - 4 miss.
 //
-// budget > 0: a ray that took that many rounds and is in no block stops: the
-// march returns kRayDeferred and leaves its state in *st (march_group resumes
-// it).
+// budget > 0: a ray that took that many rounds and is in no block and short of
+// d_max stops: the march returns kRayDeferred and leaves its state in *st
+// (march_group resumes it).
 //
 // Bound by VALU issue and the rounds of a wavefront's slowest ray.  As three
 // nested loops the same rounds took 109 us of k_raycast at 848 x 480 in the
@@ -1025,6 +1025,9 @@ __host__ __device__ RayResult march(const GridView& g, const Pose& pose, const R
                     phase = kAdvance;
                     first = true;
                     have = false;
+                    // (with d_trunc > vbl that goes forward, past d_max perhaps,
+                    // where the march makes one lookup more and ends: not deferred)
+                    rounds = l < dmax ? rounds : -(1 << 30);
                 } else {
                     vb3(rv, rp, bx, by, bz);
                     cur = id;

@@ -52,9 +52,8 @@ def scene(request):
     return o, cfg, intr, [synth.pose_f32(T) for T in views], H, W
 
 
-@pytest.mark.parametrize("budget", [0, 1, 2, 5, 12])
-def test_far_bound_and_deferred_state(lib, scene, budget):
-    o, cfg, intr, views, H, W = scene
+def raycasts(lib, o, cfg, intr, views, H, W, budget, dmax=10.0):
+    """Compares every view's march with the oracle's; returns the summed counts."""
     ex = o.export()
     n = len(ex["keys"])
     nb = 1 << max(10, (2 * n).bit_length())
@@ -64,11 +63,18 @@ def test_far_bound_and_deferred_state(lib, scene, budget):
         pts, dep, ub = np.zeros((H, W, 3), np.float32), np.zeros((H, W), np.float32), np.zeros((H, W), np.uint8)
         c = np.zeros(8, np.uint64)
         assert lib.march_far_host(H, W, f(intr[0]), f(intr[1]), f(intr[2]), f(intr[3]), f(cfg["voxel_length"]),
-                                  f(cfg["truncation"]), f(10.0), n, ex["keys"].ctypes.data, ex["coords"].ctypes.data,
+                                  f(cfg["truncation"]), f(dmax), n, ex["keys"].ctypes.data, ex["coords"].ctypes.data,
                                   ex["sdf"].ctypes.data, ex["w"].ctypes.data, C.c_uint32(nb), E.ctypes.data, budget,
                                   pts.ctypes.data, dep.ctypes.data, ub.ctypes.data, c.ctypes.data) == 0
         compare((pts, dep, ub, int(c[0]), int(c[1])), o.raycast(E.reshape(4, 4)))
         total += c
+    return total
+
+
+@pytest.mark.parametrize("budget", [0, 1, 2, 5, 12])
+def test_far_bound_and_deferred_state(lib, scene, budget):
+    o, cfg, intr, views, H, W = scene
+    total = raycasts(lib, o, cfg, intr, views, H, W, budget)
     # the far bound saves lookups where rays leave the map (none do in the room's first frames)
     assert total[2] < total[3] or (cfg is synth.ROOM_LARGE and total[2] == total[3])
     deferred, in_skip, in_advance, ahead = (int(x) for x in total[4:8])
@@ -77,6 +83,26 @@ def test_far_bound_and_deferred_state(lib, scene, budget):
           f"{ahead} with a lookup ahead")
     if cfg is synth.PLAIN_SMALL and 0 < budget < 5:
         assert in_skip and in_advance and ahead  # every kind of state
+
+
+@pytest.mark.parametrize("budget", [1, 2, 3, 5])
+@pytest.mark.parametrize("blocks", [1.125, 1.5])
+def test_truncation_beyond_the_block(lib, blocks, budget):
+    """With d_trunc > vbl the step back before a re-advance goes forward, past
+    d_max where a ray hits its first block just before it: the re-advance still
+    makes (and counts) its first lookup, and such a ray is not deferred."""
+    H, W = 97, 131
+    cfg = dict(synth.PLAIN_SMALL, voxel_length=0.01, truncation=0.08 * blocks)
+    intr = synth.scaled_intr(cfg, H, W)
+    poses = synth.traj_plain_small(n=12)[:3]
+    depth = synth.frames(synth.scene_plain_small(), poses, dict(cfg, intr=intr), seed=3, H=H, W=W)
+    for dmax in (1.0, 1.2, 1.5, 1.8):
+        o = oracle.OracleGrid(cfg["voxel_length"], cfg["truncation"], H, W, max_ray_length=dmax)
+        o.set_intrinsics(*intr)
+        for d, T in zip(depth, poses):
+            o.integrate(d, synth.pose_f32(T))
+        assert raycasts(lib, o, cfg, intr, [synth.pose_f32(T) for T in poses], H, W, budget, dmax)[4] > 0
+        o.close()
 
 
 def test_rule_of_the_budget(lib):
